@@ -233,7 +233,8 @@ struct LnChain {
 // finish sooner, one forward at a time).
 static bool small_rows(long long rows) { return rows < 2 * 256 * 64; }
 
-// Images per batch from which the attention kernel runs the QKV GEMM.
+// Images per batch from which hv_block_forward's attention kernel runs the
+// QKV GEMM (the model's does at every batch size).
 static constexpr int kFusedQkvMinBatch = 32;
 
 // transformer_block (transformer.py:401-431) on rows [0, offsets[batch]):
@@ -241,11 +242,16 @@ static constexpr int kFusedQkvMinBatch = 32;
 // warnings (optional, [B]) receive the LayerNorms' negative-variance bit.
 // bias_max (optional, device): the largest |bias| of bqkv, bproj, b1 and b2.
 // ffn_rows: the fused FFN's row blocking (FfnRows, launch_ffn).
+// check: the per-image status and cleared warnings, written by the attention
+// kernel (hv_block_forward without a separate image check).
+struct ImageCheck {
+  int32_t *status, *warnings;
+};
 static int block_forward(const hv_block_dev &p, const int8_t *x, const int32_t *offsets,
                          int batch, int max_rows, int8_t *z, const hv_block_ckpt *ck,
                          int32_t *warnings, const BlockWs &w, hipStream_t s,
                          const LnChain &chain = LnChain{}, const unsigned *bias_max = nullptr,
-                         int ffn_rows = FFN_ROWS64) {
+                         int ffn_rows = FFN_ROWS64, const ImageCheck &check = ImageCheck{}) {
   const int32_t *rows_dev = offsets + batch;
   const LnWarn lw{offsets, batch, warnings};
   int8_t *qkv = ck && ck->fused_qkv ? ck->fused_qkv : w.qkv;
@@ -274,11 +280,13 @@ static int block_forward(const hv_block_dev &p, const int8_t *x, const int32_t *
   g.shift_a = p.qkv_out_exp - (p.ln1_out_exp + p.wqkv_exp);
   // Without checkpoints the attention kernel computes each head's Q, K and
   // V itself when their requant takes the int32 form: qkv never reaches
-  // memory.  Small batches keep the separate GEMM: with a few workgroups
-  // per head the in-kernel GEMM would run on a few CUs in series with the
-  // attention (one image: 0.63 ms → 0.67 ms per forward).
+  // memory, and a launch is saved (one image, unpruned forward: 288 us with
+  // it in the kernel, 309 us with the separate GEMM).  A block call of few
+  // images has no tensor-wide bias bound, so its in-kernel requant would vote
+  // tile by tile, and keeps the separate GEMM (one image: 27.0 us, 25.7 us
+  // in the kernel).
   epilogue_limits_pub(g, HV_EPI_I8);
-  const bool fuse_qkv = !ck && batch >= kFusedQkvMinBatch && g.narrow_ok && g.shift_a >= -30 &&
+  const bool fuse_qkv = !ck && (bias_max || batch >= kFusedQkvMinBatch) && g.narrow_ok && g.shift_a >= -30 &&
                         g.shift_a <= 30 &&
                         !(((uintptr_t)ln1 | (uintptr_t)p.wqkv_p | (uintptr_t)p.bqkv) & 15);
   if (!fuse_qkv) {
@@ -293,6 +301,7 @@ static int block_forward(const hv_block_dev &p, const int8_t *x, const int32_t *
     a.qkv_shift = g.shift_a; a.qkv_acc_lim = g.acc_lim; a.bqkv_max = bias_max;
   }
   a.qkv = qkv; a.offsets = offsets; a.ctx = ctx; a.batch = batch; a.rows_cap = max_rows;
+  a.status = check.status; a.warnings = check.warnings;
   a.score = ck ? ck->score : nullptr;
   a.prob = ck ? ck->prob : nullptr;
   a.score_shift = p.score_exp - 2 * p.qkv_out_exp;
@@ -447,10 +456,9 @@ int hv_attention_i8(const int8_t *qkv, const int32_t *offsets, int batch, int ro
     return fail(HV_EVALUE, HV_ERR_ADDRESS,
                 "attention: qkv must be 16-byte and ctx 4-byte aligned");
   const hipStream_t s = (hipStream_t)stream;
-  int rc = launch_image_check(offsets, batch, rows, status, nullptr, s);
-  if (rc) return rc;
   AttnArgs a{};
   a.qkv = qkv; a.offsets = offsets; a.ctx = ctx; a.batch = batch; a.rows_cap = rows;
+  a.status = status;
   a.score = score; a.prob = prob;
   a.score_shift = score_exp - 2 * qkv_exp;
   a.q16_shift = -(score_exp + 13);
@@ -504,11 +512,24 @@ int hv_block_forward(const hv_block_dev *p, const int8_t *x, const int32_t *offs
   Carve cv{(uint8_t *)workspace, workspace_bytes};
   BlockWs w = carve_block(cv, (size_t)max_rows);
   if (!cv.ok || !workspace) return fail(HV_EVALUE, HV_ERR_ADDRESS, "block: workspace too small");
-  if ((rc = launch_image_check(offsets, batch, max_rows, status, warnings, (hipStream_t)stream)))
+  // With both LayerNorms in the int32 form, which never finds a negative
+  // variance, nothing sets a warning bit: the attention kernel then writes
+  // the status and clears the warnings, and the check needs no launch of its
+  // own (1.4-3.9 us with the gap behind it; one image 27.0 -> 24.6 us).
+  Ln32 ln;
+  const bool in_attention =
+      ((uintptr_t)x & 7) == 0 &&
+      ln32_setup(p->ln1_gamma, p->ln1_beta, ck && ck->ln1 ? ck->ln1 : w.ln, p->x_exp,
+                 p->gamma1_exp, p->beta1_exp, p->ln1_out_exp, &ln) &&
+      ln32_setup(p->ln2_gamma, p->ln2_beta, ck && ck->ln2 ? ck->ln2 : w.ln, p->ffn_x_exp,
+                 p->gamma2_exp, p->beta2_exp, p->ln2_out_exp, &ln);
+  const ImageCheck check = in_attention ? ImageCheck{status, warnings} : ImageCheck{};
+  if (!in_attention && (rc = launch_image_check(offsets, batch, max_rows, status, warnings,
+                                                (hipStream_t)stream)))
     return rc;
   return block_forward(*p, x, offsets, batch, max_rows, z, ck, warnings, w, (hipStream_t)stream,
                        LnChain{}, nullptr,
-                       small_rows(max_rows) ? FFN_ROWS32 : FFN_ROWS64_BALANCED);
+                       small_rows(max_rows) ? FFN_ROWS32 : FFN_ROWS64_BALANCED, check);
 }
 
 struct SelectorWs {

@@ -1515,9 +1515,9 @@ static void launch_ffn_d(const GemmArgs &g1, const GemmArgs &g2, const LnPrologu
 }
 
 // CUs of the current device (cached per device; host threads may race to
-// fill an entry, all with the same value).  It only places the split of
-// ffn_full_blocks: any split gives the same outputs.
-static int device_cus() {
+// fill an entry, all with the same value).  It only places the splits of
+// ffn_full_blocks and launch_attention: any split gives the same outputs.
+int device_cus() {
   static std::atomic<int> cus[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

@@ -160,6 +160,8 @@ struct AttnArgs {
   int q16_mode, q16_s, q16_rnd;  // int32 fast path for the score -> Q8.16 conversion
   int ctx_fast, ctx_rnd;         // int32 context requant (shift in [1, 30])
   int rows_cap;                  // rows of qkv / ctx; images outside are skipped
+  int32_t *status;    // optional [B]: HV_ERR_TOKEN_COUNT for a skipped image, else 0
+  int32_t *warnings;  // optional [B]: set to 0
   // Fused QKV (ln1 non-NULL): each head's Q, K and V come from the kernel's
   // own GEMM over the LayerNorm 1 rows (row stride 192, the same row
   // offsets), qkv unused.  wqkv mfma32-packed [192][576]; the int8 requant
@@ -169,6 +171,7 @@ struct AttnArgs {
   const int8_t *wqkv;
   const int32_t *bqkv;
   int qkv_shift, qkv_acc_lim;
+  int q_split;  // workgroups per (image, head), each a range of its query tiles
   const unsigned *bqkv_max;  // optional: largest |bias| of bqkv (GemmArgs::bias_max)
 };
 
@@ -178,6 +181,8 @@ __device__ __forceinline__ bool tensor_narrow(const unsigned *bias_max, int acc_
   return bias_max && acc_lim > 0 && *bias_max <= (unsigned)acc_lim;
 }
 int launch_attention(const AttnArgs &a, hipStream_t s);
+// CUs of the current device (hv_gemm.hip).
+int device_cus();
 
 int launch_softmax_rows(const int32_t *x, const int32_t *offsets, int rows, uint8_t *att,
                         int32_t *sel, hipStream_t s);

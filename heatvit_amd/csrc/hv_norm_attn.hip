@@ -413,51 +413,44 @@ __device__ __forceinline__ void qkv_load_a(v4i (&a)[6], const int8_t *rows) {
 // -128 V[k] + 128 V[k] = 0 whatever its V, its K row only meets masked
 // scores, and Q rows from N on are never read.
 template <bool LA, bool NARROW, bool ISV>
-__device__ __forceinline__ void qkv_unit(const AttnArgs &g, const v4i (&w)[2][6],
-                                         const v4i (&a)[6], int p, int rt, int8_t *Qs,
-                                         int8_t *Ks, int8_t *Vt, int *vsum, const int *bias_s,
-                                         int rows_k, int lane, const Rq &rq) {
+__device__ __forceinline__ void qkv_tile(const AttnArgs &g, const v4i (&w)[6], const v4i (&a)[6],
+                                         int p, int c, int rt, int8_t *Qs, int8_t *Ks, int8_t *Vt,
+                                         int *vsum, const int *bias_s, int rows_k, int lane,
+                                         const Rq &rq) {
   const int l32 = lane & 31, hh = lane >> 5;
   if constexpr (ISV) {
     // channel of this lane's column under the weight packing
     const int pj = 16 * ((l32 >> 2) & 1) + 4 * (l32 >> 3) + (l32 & 3);
+    v16i acc = v16i{0};
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      v16i acc = v16i{0};
+    for (int kt = 0; kt < 6; ++kt)
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kt], w[kt], acc, 0, 0, 0);
+    const int bias = bias_s[128 + c * 32 + pj];
+    if (NARROW || __all(bias <= g.qkv_acc_lim && bias >= -g.qkv_acc_lim)) {
 #pragma unroll
-      for (int kt = 0; kt < 6; ++kt)
-        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[kt], w[c][kt], acc, 0, 0, 0);
-      const int bias = bias_s[128 + c * 32 + pj];
-      if (NARROW || __all(bias <= g.qkv_acc_lim && bias >= -g.qkv_acc_lim)) {
+      for (int j = 0; j < 16; ++j) acc[j] = rq_dir_nowrap<LA>(acc[j] + bias, rq);
+    } else {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] = rq_dir_nowrap<LA>(acc[j] + bias, rq);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 16; ++j) acc[j] = attn_requant8(acc[j], bias, g.qkv_shift);
-      }
-      int8_t *vrow = Vt + (c * 32 + pj) * kVStride;
-      int vs = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int t0 = rt * 32 + 8 * k + 4 * hh;  // keys t0 .. t0 + 3
-        const unsigned wd = pack_lo4(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
-        vs = __builtin_amdgcn_sdot4((int)wd, 0x01010101, vs, false);
-        *reinterpret_cast<unsigned *>(vrow + vt_pos(t0)) = wd;
-      }
-      atomicAdd(&vsum[c * 32 + pj], vs * 128);
-      __builtin_amdgcn_sched_barrier(0);  // one column tile's registers at a time
+      for (int j = 0; j < 16; ++j) acc[j] = attn_requant8(acc[j], bias, g.qkv_shift);
     }
-    return;
-  }
-  const int r = rt * 32 + l32;
+    int8_t *vrow = Vt + (c * 32 + pj) * kVStride;
+    int vs = 0;
 #pragma unroll
-  for (int c = 0; c < 2; ++c) {
+    for (int k = 0; k < 4; ++k) {
+      const int t0 = rt * 32 + 8 * k + 4 * hh;  // keys t0 .. t0 + 3
+      const unsigned wd = pack_lo4(acc[4 * k], acc[4 * k + 1], acc[4 * k + 2], acc[4 * k + 3]);
+      vs = __builtin_amdgcn_sdot4((int)wd, 0x01010101, vs, false);
+      *reinterpret_cast<unsigned *>(vrow + vt_pos(t0)) = wd;
+    }
+    atomicAdd(&vsum[c * 32 + pj], vs * 128);
+  } else {
+    const int r = rt * 32 + l32;
     // this lane's 16 channels c*32 + 16*hh + j
     const int *bc = bias_s + p * 64 + c * 32 + 16 * hh;
     v16i acc = NARROW ? *reinterpret_cast<const v16i *>(bc) : v16i{0};
 #pragma unroll
     for (int kt = 0; kt < 6; ++kt)
-      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[c][kt], a[kt], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[kt], a[kt], acc, 0, 0, 0);
     v4i o;
     if (NARROW) {
 #pragma unroll
@@ -473,8 +466,18 @@ __device__ __forceinline__ void qkv_unit(const AttnArgs &g, const v4i (&w)[2][6]
     }
     const int ch = c * 32 + 16 * hh;  // channel within the head
     if (r < rows_k) *reinterpret_cast<v4i *>(&(p == 0 ? Qs : Ks)[r * kKStride + ch]) = o;
-    __builtin_amdgcn_sched_barrier(0);  // one column tile's registers at a time
   }
+  __builtin_amdgcn_sched_barrier(0);  // one column tile's registers at a time
+}
+
+template <bool LA, bool NARROW, bool ISV>
+__device__ __forceinline__ void qkv_unit(const AttnArgs &g, const v4i (&w)[2][6],
+                                         const v4i (&a)[6], int p, int rt, int8_t *Qs,
+                                         int8_t *Ks, int8_t *Vt, int *vsum, const int *bias_s,
+                                         int rows_k, int lane, const Rq &rq) {
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    qkv_tile<LA, NARROW, ISV>(g, w[c], a, p, c, rt, Qs, Ks, Vt, vsum, bias_s, rows_k, lane, rq);
 }
 
 // Wavefront p < 3 runs group p (0 Q, 1 K, 2 V) over all its row tiles
@@ -516,6 +519,64 @@ __device__ __forceinline__ void qkv_units(const AttnArgs &g, const v4i (&w)[2][6
     qkv_rows<LA, NARROW, false>(g, w, wave, Qs, Ks, Vt, vsum, bias_s, row0, N, lane);
 }
 
+// One column tile (32 channels, weights w) of group p over row tiles rt0,
+// rt0 + step, ... below rt1; the next tile's A rows load while the current
+// one multiplies.
+template <bool LA, bool NARROW, bool ISV>
+__device__ __forceinline__ void qkv_cols(const AttnArgs &g, const v4i (&w)[6], int p, int c,
+                                         int rt0, int rt1, int step, int8_t *Qs, int8_t *Ks,
+                                         int8_t *Vt, int *vsum, const int *bias_s, int row0, int N,
+                                         int lane) {
+  if (rt0 >= rt1) return;
+  const int rows_k = ((N + 15) >> 4) * 16;
+  const Rq rq = rq_setup(g.qkv_shift, -128, 127);
+  const int8_t *ln1 = g.ln1 + (size_t)row0 * 192 + 16 * (lane >> 5);
+  auto a_rows = [&](int rt) {
+    return ln1 + (size_t)min(min(rt, rt1 - 1) * 32 + (lane & 31), N - 1) * 192;
+  };
+  v4i a0[6], a1[6];
+  qkv_load_a(a0, a_rows(rt0));
+#pragma unroll 1
+  for (int rt = rt0; rt < rt1; rt += 2 * step) {
+    qkv_load_a(a1, a_rows(rt + step));
+    qkv_tile<LA, NARROW, ISV>(g, w, a0, p, c, rt, Qs, Ks, Vt, vsum, bias_s, rows_k, lane, rq);
+    if (rt + step >= rt1) break;
+    qkv_load_a(a0, a_rows(rt + 2 * step));
+    qkv_tile<LA, NARROW, ISV>(g, w, a1, p, c, rt + step, Qs, Ks, Vt, vsum, bias_s, rows_k, lane,
+                              rq);
+  }
+}
+
+// Eight wavefronts: wavefront w takes one column tile of K (w % 4 < 2) or V
+// over every second row tile, then column tile w % 2 of Q over the row tiles
+// of its workgroup's queries [q0, q1) (16-query tiles), every fourth one
+// (the wavefronts with fewer K and V tiles first).  wk: the K or V weights.
+template <bool LA, bool NARROW>
+__device__ __forceinline__ void qkv_wide(const AttnArgs &g, const v4i (&wk)[6], int8_t *Qs,
+                                         int8_t *Ks, int8_t *Vt, int *vsum, const int *bias_s,
+                                         int row0, int N, int h, int q0, int q1, int wave,
+                                         int lane) {
+  const int c = wave & 1, half = wave >> 2;
+  v4i wq[6];
+  qkv_load_w(wq, g.wqkv, h * 2 + c, lane);
+  if (wave & 2)
+    qkv_cols<LA, NARROW, true>(g, wk, 2, c, half, (N + 31) >> 5, 2, Qs, Ks, Vt, vsum, bias_s,
+                               row0, N, lane);
+  else
+    qkv_cols<LA, NARROW, false>(g, wk, 1, c, half, ((N + 15) / 16 + 1) >> 1, 2, Qs, Ks, Vt, vsum,
+                                bias_s, row0, N, lane);
+  qkv_cols<LA, NARROW, false>(g, wq, 0, c, (q0 >> 1) + (((wave >> 1) + 2) & 3), (q1 + 1) >> 1, 4,
+                              Qs, Ks, Vt, vsum, bias_s, row0, N, lane);
+}
+
+// keys of the last 64-key chunk past the V tiles: zero (four keys of one
+// channel per dword)
+__device__ __forceinline__ void zero_tail_keys(int8_t *Vt, int N) {
+  const int nv = (N + 31) >> 5, kz = nv * 32, runs = (((N + 63) >> 6) * 64 - kz) >> 2;
+  for (int i = threadIdx.x; i < runs * 64; i += blockDim.x)
+    *reinterpret_cast<unsigned *>(Vt + (i & 63) * kVStride + vt_pos(kz + 4 * (i >> 6))) = 0u;
+}
+
 template <bool LA>
 __device__ __forceinline__ void qkv_head(const AttnArgs &g, const v4i (&w)[2][6], int8_t *Qs,
                                          int8_t *Ks, int8_t *Vt, int *vsum, const int *bias_s,
@@ -524,28 +585,25 @@ __device__ __forceinline__ void qkv_head(const AttnArgs &g, const v4i (&w)[2][6]
     qkv_units<LA, true>(g, w, Qs, Ks, Vt, vsum, bias_s, row0, N, wave, lane);
   else
     qkv_units<LA, false>(g, w, Qs, Ks, Vt, vsum, bias_s, row0, N, wave, lane);
-  // keys of the last 64-key chunk past the V tiles: zero (four keys of one
-  // channel per dword)
-  const int nv = (N + 31) >> 5, kz = nv * 32, runs = (((N + 63) >> 6) * 64 - kz) >> 2;
-  for (int i = threadIdx.x; i < runs * 64; i += blockDim.x)
-    *reinterpret_cast<unsigned *>(Vt + (i & 63) * kVStride + vt_pos(kz + 4 * (i >> 6))) = 0u;
+  zero_tail_keys(Vt, N);
 }
 
 // The query tiles of one wavefront for an image of NT key tiles (N in
 // (16 (NT - 1), 16 NT]): straight-line code per tile count, so the score
 // MFMAs issue back to back and only the last tile masks padded keys.
 // FQ: the queries come from Qs in LDS (fused QKV), else from qkv.
-template <int MODE, bool CKPT, int NT, bool FQ>
+template <int MODE, bool CKPT, int NT, bool FQ, int NW>
 __device__ __forceinline__ void attn_tiles(const AttnArgs &g, const int8_t *Ks, const int8_t *Vt,
                                            const int *vsum, const int8_t *qkv, const int8_t *Qs,
-                                           int b, int h, int N, int row0, int wave, int lane) {
+                                           int b, int h, int N, int row0, int q0, int q1, int wave,
+                                           int lane) {
   constexpr int NC = (NT + 3) / 4;  // PV chunks of 64 keys
   const int ql = lane & 15, grp = lane >> 4;
   const int kvalid = N - 16 * (NT - 1) - 4 * grp;  // valid keys i < kvalid in the last tile
   // Query tiles round-robin over the wavefronts, rotated by workgroup so
   // the wavefront that gets the extra tile sits on a different SIMD in
   // neighbouring workgroups.
-  for (int qt = (wave + blockIdx.x) & 3; qt < NT; qt += 4) {
+  for (int qt = q0 + ((wave + blockIdx.x) & (NW - 1)); qt < q1; qt += NW) {
     const int q = qt * 16 + ql;  // this lane's query
     v4i qb = v4i{0};
     if (q < N)
@@ -662,8 +720,9 @@ __device__ __forceinline__ void attn_tiles(const AttnArgs &g, const int8_t *Ks, 
 // At most 168 VGPRs (three workgroups per CU): the 768 items of a 256-image
 // batch then run in one round.  FQ: fused QKV (qkv_head), FQL its requant
 // shifting left.
-template <int MODE, bool CKPT, bool FQ, bool FQL>
-__global__ __launch_bounds__(256, 3) void k_attention(AttnArgs g) {
+template <int MODE, bool CKPT, bool FQ, bool FQL, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 2) void k_attention(AttnArgs g) {
+  constexpr int NTH = 64 * NW;
   __shared__ __attribute__((aligned(16))) int8_t Ks[kMaxKeys * kKStride];
   __shared__ __attribute__((aligned(16))) int8_t Vt[64 * kVStride];
   __shared__ __attribute__((aligned(16))) int vsum[64];  // 128 * sum_k V[k][d]
@@ -674,17 +733,20 @@ __global__ __launch_bounds__(256, 3) void k_attention(AttnArgs g) {
   // The grid is a multiple of 8 and workgroups go round-robin over the 8
   // XCDs, so XCD x runs logical items [x*T8, (x+1)*T8): the three heads of
   // an image share one XCD's L2 and each row of QKV is fetched once.
-  const int T = 3 * g.batch, T8 = (T + 7) >> 3;
+  const int T = 3 * g.batch * g.q_split, T8 = (T + 7) >> 3;
   const int L = (blockIdx.x & 7) * T8 + (blockIdx.x >> 3);
   if (L >= T) return;
-  const int b = L / 3, h = L - 3 * b;
+  const int item = NW == 4 ? L : L / g.q_split, part = L - item * g.q_split;
+  const int b = item / 3, h = item - 3 * b;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // FQ: wavefront p < 3's weight fragments of Q, K or V and the head's
   // biases load before the row offsets, whose latency they share
-  v4i w[2][6];
+  v4i w[NW == 4 ? 2 : 1][6];
   int bias_v = 0;
   if constexpr (FQ) {
-    if (wave < 3) {
+    if constexpr (NW == 8) {
+      qkv_load_w(w[0], g.wqkv, ((wave & 2) ? 12 : 6) + h * 2 + (wave & 1), lane);
+    } else if (wave < 3) {
       qkv_load_w(w[0], g.wqkv, wave * 6 + h * 2, lane);
       qkv_load_w(w[1], g.wqkv, wave * 6 + h * 2 + 1, lane);
     }
@@ -693,26 +755,43 @@ __global__ __launch_bounds__(256, 3) void k_attention(AttnArgs g) {
   const int row0 = g.offsets[b];
   const int N = g.offsets[b + 1] - row0;
   // Images with a token count outside [1, 197] or rows outside the
-  // buffers are skipped (reported by the block's image check).
-  if (N <= 0 || N > HV_MAX_TOKENS || row0 < 0 || row0 > g.rows_cap - N) return;
+  // buffers are skipped.
+  const bool ok = N >= 1 && N <= HV_MAX_TOKENS && row0 >= 0 && row0 <= g.rows_cap - N;
+  if (h == 0 && part == 0 && tid == 0) {
+    if (g.status) g.status[b] = ok ? HV_ERR_NONE : HV_ERR_TOKEN_COUNT;
+    if (g.warnings) g.warnings[b] = 0;
+  }
+  if (!ok) return;
   const int n16 = (N + 15) >> 4;  // key / query tiles
   const int n64 = (N + 63) >> 6;  // PV chunks of 64 keys
   const int8_t *qkv = FQ ? nullptr : g.qkv + (size_t)row0 * 576;
+  // this workgroup's query tiles [q0, q1) of the image's n16
+  const int q0 = NW == 4 ? 0 : part * n16 / g.q_split;
+  const int q1 = NW == 4 ? n16 : (part + 1) * n16 / g.q_split;
+  if (q0 >= q1) return;  // uniform
 
   if constexpr (FQ) {
     if (tid < 64) vsum[tid] = 0;
     if (tid < 192) bias_s[tid] = bias_v;
     __syncthreads();
-    qkv_head<FQL>(g, w, Qs, Ks, Vt, vsum, bias_s, row0, N, wave, lane);
+    if constexpr (NW == 8) {
+      if (tensor_narrow(g.bqkv_max, g.qkv_acc_lim))
+        qkv_wide<FQL, true>(g, w[0], Qs, Ks, Vt, vsum, bias_s, row0, N, h, q0, q1, wave, lane);
+      else
+        qkv_wide<FQL, false>(g, w[0], Qs, Ks, Vt, vsum, bias_s, row0, N, h, q0, q1, wave, lane);
+      zero_tail_keys(Vt, N);
+    } else {
+      qkv_head<FQL>(g, w, Qs, Ks, Vt, vsum, bias_s, row0, N, wave, lane);
+    }
   } else {
-  for (int i = tid; i < n16 * 16 * 4; i += 256) {
+  for (int i = tid; i < n16 * 16 * 4; i += NTH) {
     const int r = i >> 2, c = (i & 3) * 16;
     v4i v = v4i{0};
     if (r < N) v = *reinterpret_cast<const v4i *>(qkv + (size_t)r * 576 + 192 + h * 64 + c);
     *reinterpret_cast<v4i *>(&Ks[r * kKStride + c]) = v;
   }
   // V^T: item (key quad kq, 16-channel group dg); keys beyond N are zero.
-  for (int i = tid; i < n64 * 64; i += 256) {
+  for (int i = tid; i < n64 * 64; i += NTH) {
     const int kq = i >> 2, dg = i & 3;
     v4i rows[4];
 #pragma unroll
@@ -751,7 +830,8 @@ __global__ __launch_bounds__(256, 3) void k_attention(AttnArgs g) {
 
   switch (n16) {
 #define HV_ATTN_CASE(n) \
-    case n: attn_tiles<MODE, CKPT, n, FQ>(g, Ks, Vt, vsum, qkv, Qs, b, h, N, row0, wave, lane); \
+    case n: attn_tiles<MODE, CKPT, n, FQ, NW>(g, Ks, Vt, vsum, qkv, Qs, b, h, N, row0, q0, q1, \
+                                              wave, lane); \
       break;
     HV_ATTN_CASE(1) HV_ATTN_CASE(2) HV_ATTN_CASE(3) HV_ATTN_CASE(4) HV_ATTN_CASE(5)
     HV_ATTN_CASE(6) HV_ATTN_CASE(7) HV_ATTN_CASE(8) HV_ATTN_CASE(9) HV_ATTN_CASE(10)
@@ -759,6 +839,29 @@ __global__ __launch_bounds__(256, 3) void k_attention(AttnArgs g) {
 #undef HV_ATTN_CASE
     default: break;
   }
+}
+
+template <int NW>
+static void launch_attention_mode(const AttnArgs &a, hipStream_t s) {
+  const dim3 grid((a.batch * 3 * a.q_split + 7) / 8 * 8), block(64 * NW);
+  const bool left = a.qkv_shift <= 0;
+  auto go = [&](auto k) { hv_launch(k, grid, block, 0, s, a); };
+  switch (a.q16_mode * 2 + (left ? 1 : 0)) {
+    case 0: go(k_attention<0, false, true, false, NW>); break;
+    case 1: go(k_attention<0, false, true, true, NW>); break;
+    case 2: go(k_attention<1, false, true, false, NW>); break;
+    case 3: go(k_attention<1, false, true, true, NW>); break;
+    case 4: go(k_attention<2, false, true, false, NW>); break;
+    default: go(k_attention<2, false, true, true, NW>); break;
+  }
+}
+
+template <int NW>
+static void launch_attention_plain(const AttnArgs &a, hipStream_t s) {
+  const dim3 grid((a.batch * 3 * a.q_split + 7) / 8 * 8), block(64 * NW);
+  if (a.q16_mode == 0) hv_launch((k_attention<0, false, false, false, NW>), grid, block, 0, s, a);
+  else if (a.q16_mode == 1) hv_launch((k_attention<1, false, false, false, NW>), grid, block, 0, s, a);
+  else hv_launch((k_attention<2, false, false, false, NW>), grid, block, 0, s, a);
 }
 
 int launch_attention(const AttnArgs &a_in, hipStream_t s) {
@@ -786,30 +889,41 @@ int launch_attention(const AttnArgs &a_in, hipStream_t s) {
   a.ctx_fast = a.ctx_shift >= 1 && a.ctx_shift <= 30;
   a.ctx_rnd = a.ctx_fast ? 1 << (a.ctx_shift - 1) : 0;
   const bool ck = a.score || a.prob;
-  const dim3 grid((a.batch * 3 + 7) / 8 * 8), block(256);
+  // Few (image, head) pairs leave CUs idle and a pair's tiles in series on
+  // four wavefronts, so they run on workgroups of eight, and with fewer pairs
+  // than half the CUs on two to four workgroups each, every one a range of
+  // the query tiles (K and V are computed or loaded again in each).  Beyond
+  // one workgroup per CU the repeated K and V cost more than the split gives:
+  // fused QKV, unpruned forward on MI355X, four waves / eight / eight split in
+  // two / in four (us):
+  //    1 image 385 / 352 / 306 / 288    24 images 389 / 357 / 310 / 358
+  //   42       460 / 428 / 384 / 432    64        472 / 441 / 491 / 511
+  //   85       584 / 551 / 602 / 685   100        654 / 692 / 707 / 760
+  // Over given QKV rows K and V are only loaded, and two parts stay ahead up
+  // to 1.5 pairs per CU (96 ragged images 16.2 / 14.8 / 14.3 / 16.4, 128:
+  // 19.3 / 19.3 / 18.0 / 20.2, 256: 22.9 / 23.3 / 26.4 / 32.0).
+  const int items = a.batch * 3, cus = device_cus();
+  const bool wide = a.ln1 ? items <= cus : 2 * items <= 3 * cus;
+  const int nw = wide ? 8 : 4, per_cu = cus / items;
+  a.q_split = !wide ? 1 : (a.ln1 ? min(max(per_cu, 1), 4) : (per_cu >= 4 ? 4 : 2));
   if (a.ln1) {
     // fused QKV: no checkpoints, the int32-form shift range
     if (ck || !a.wqkv || !a.bqkv || a.qkv_shift < -30 || a.qkv_shift > 30 ||
         (((uintptr_t)a.ln1 | (uintptr_t)a.wqkv | (uintptr_t)a.bqkv) & 15))
       return fail(HV_EVALUE, HV_ERR_DIMENSION, "attention: fused QKV arguments");
-    const bool left = a.qkv_shift <= 0;
-    auto go = [&](auto k) { hv_launch(k, grid, block, 0, s, a); };
-    switch (a.q16_mode * 2 + (left ? 1 : 0)) {
-      case 0: go(k_attention<0, false, true, false>); break;
-      case 1: go(k_attention<0, false, true, true>); break;
-      case 2: go(k_attention<1, false, true, false>); break;
-      case 3: go(k_attention<1, false, true, true>); break;
-      case 4: go(k_attention<2, false, true, false>); break;
-      default: go(k_attention<2, false, true, true>); break;
-    }
-    return check_hip(hipGetLastError(), "k_attention launch");
+    if (nw == 8) launch_attention_mode<8>(a, s);
+    else launch_attention_mode<4>(a, s);
+  } else if (ck) {
+    a.q_split = 1;
+    const dim3 grid((items + 7) / 8 * 8), block(256);
+    if (a.q16_mode == 0) hv_launch((k_attention<0, true, false, false, 4>), grid, block, 0, s, a);
+    else if (a.q16_mode == 1) hv_launch((k_attention<1, true, false, false, 4>), grid, block, 0, s, a);
+    else hv_launch((k_attention<2, true, false, false, 4>), grid, block, 0, s, a);
+  } else if (nw == 8) {
+    launch_attention_plain<8>(a, s);
+  } else {
+    launch_attention_plain<4>(a, s);
   }
-  if (a.q16_mode == 0 && !ck) hv_launch((k_attention<0, false, false, false>), grid, block, 0, s, a);
-  else if (a.q16_mode == 0) hv_launch((k_attention<0, true, false, false>), grid, block, 0, s, a);
-  else if (a.q16_mode == 1 && !ck) hv_launch((k_attention<1, false, false, false>), grid, block, 0, s, a);
-  else if (a.q16_mode == 1) hv_launch((k_attention<1, true, false, false>), grid, block, 0, s, a);
-  else if (!ck) hv_launch((k_attention<2, false, false, false>), grid, block, 0, s, a);
-  else hv_launch((k_attention<2, true, false, false>), grid, block, 0, s, a);
   return check_hip(hipGetLastError(), "k_attention launch");
 }
 

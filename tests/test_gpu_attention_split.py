@@ -1,0 +1,77 @@
+"""GPU parity of the attention kernel's work splits: four or eight wavefronts
+per workgroup and one to four workgroups per (image, head), chosen from the
+image count.  The batches sit on both sides of each change of split on a
+256-CU device and their images at the edges of the 16-query and 32-row tiles
+(images with fewer query tiles than workgroups among them); every output is
+compared with the CPU oracle, bit for bit."""
+
+import numpy as np
+import pytest
+
+from heatvit_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+EDGES = (197, 1, 16, 17, 32, 33, 48, 63, 64, 65, 96, 128, 129, 192, 193)
+
+
+def _lengths(batch):
+    return [EDGES[i % len(EDGES)] for i in range(batch)]
+
+
+@pytest.mark.parametrize("batch", (1, 21, 22, 128, 129))
+def test_attention_over_given_qkv(oracle, batch):
+    from heatvit_amd.ops import attention
+    from test_gpu_attention import peaky_qkv
+    rng = np.random.default_rng(batch)
+    m = synth.block_workload()[1].mhsa
+    exps = (m.qkv_out_scale_exp, m.score_scale_exp, m.prob_scale_exp, m.context_out_scale_exp)
+    qkvs = [peaky_qkv(rng, n) for n in _lengths(batch)]
+    got = _context(qkvs, exps)
+    for i, q in enumerate(qkvs):
+        want = oracle.attention(q, *exps)[2]
+        assert np.array_equal(got[i], want), (batch, i, len(q))
+
+
+def _context(qkvs, exps):
+    """The context rows of hv_attention_i8 without score and prob outputs
+    (whose launches keep four wavefronts), and its status."""
+    import torch
+
+    from heatvit_amd import _lib
+    lens = [len(q) for q in qkvs]
+    offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    qkv = torch.from_numpy(np.concatenate(qkvs)).cuda()
+    off = torch.from_numpy(offsets).cuda()
+    ctx = torch.empty((int(offsets[-1]), 192), dtype=torch.int8, device="cuda")
+    status = torch.full((len(qkvs),), -1, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.lib().hv_attention_i8(
+        qkv.data_ptr(), off.data_ptr(), len(qkvs), int(offsets[-1]), ctx.data_ptr(), None, None,
+        *exps, status.data_ptr(), torch.cuda.current_stream().cuda_stream), "attention")
+    assert not status.cpu().numpy().any()
+    host = ctx.cpu().numpy()
+    return [host[offsets[i]:offsets[i + 1]] for i in range(len(qkvs))]
+
+
+@pytest.mark.parametrize("batch", (32, 42, 43, 85, 86))
+def test_block_with_qkv_in_the_attention_kernel(oracle, batch):
+    from heatvit_amd.transformer import transformer_block_batch
+    rng = np.random.default_rng(100 + batch)
+    bp = synth.block_workload()[1]
+    xs = [rng.integers(-128, 128, (n, 192)).astype(np.int8) for n in _lengths(batch)]
+    zs = transformer_block_batch(xs, bp)
+    for i, x in enumerate(xs):
+        want, _ = oracle.transformer_block(x, bp, checkpoints=False)
+        assert np.array_equal(zs[i], want), (batch, i, len(x))
+
+
+@pytest.mark.parametrize("batch", (1, 3, 22, 43))
+def test_model_of_few_images(oracle, batch):
+    from heatvit_amd.model import HeatViTModel
+    images, params = synth.pruned_workload(batch)
+    res = HeatViTModel().infer_batch(images, params)
+    logits, counts, status, warnings = oracle.model_infer_batch(images, params, threads=8)
+    assert not status.any()
+    assert np.array_equal(res.logits, logits)
+    assert np.array_equal(res.token_counts, counts)
+    assert np.array_equal(res.warnings, warnings)
