@@ -557,18 +557,18 @@ struct LnRow {
 // with inv = 2^e io (io odd), such x exist when 2^e divides K_0 mod
 // 2^(48-s) and are x = (K_0 / 2^e) io^-1 (mod 2^(48-s-e)) (all x once
 // e >= 48 - s); tie marks a row where one of them lies in [-128, xt].
-__host__ __device__ __forceinline__ void ln_row_fill(LnRow &r, double mean, double inv, i64 c2,
-                                                     i64 low, int s) {
-  const i64 f = c2 * (1ll << (48 - s)) + (low >> s);
+__host__ __device__ __forceinline__ void ln_row_set(LnRow &r, double mean, double inv, double f,
+                                                    bool tie_row, int s) {
   r.inv = ldexp(inv, s - 48);
-  r.add = ldexp((double)f, s - 48);
-  r.addm = ldexp((double)(2 * f + 1 - (1ll << (48 - s))), s - 49);
+  r.add = ldexp(f, s - 48);
+  // (2 f + 1 - 2^(48 - s)) 2^(s - 49), an integer below 2^52 scaled: exact
+  r.addm = fma(f, ldexp(1.0, s - 48), ldexp(1.0, s - 49) - 0.5);
   const double xt = floor(ldexp(mean - 1.0, -s));
   r.xt = xt > 127.0 ? 127 : (xt < -129.0 ? -129 : (int)xt);
   r.tie = false;
-  if ((low & ((1ll << s) - 1)) == 0 && r.xt >= -128) {
+  if (tie_row && r.xt >= -128) {
     const int sh = 48 - s;
-    const u64 mm = (1ull << sh) - 1, k0 = (u64)(-f) & mm, iv = (u64)inv;
+    const u64 mm = (1ull << sh) - 1, k0 = (u64)(-(i64)f) & mm, iv = (u64)inv;
     const int e = __builtin_ctzll(iv);
     if (e >= sh) {
       r.tie = k0 == 0;
@@ -581,6 +581,11 @@ __host__ __device__ __forceinline__ void ln_row_fill(LnRow &r, double mean, doub
       r.tie = -128 + (i64)((rr + 128) & pm) <= r.xt;
     }
   }
+}
+__host__ __device__ __forceinline__ void ln_row_fill(LnRow &r, double mean, double inv, i64 c2,
+                                                     i64 low, int s) {
+  ln_row_set(r, mean, inv, (double)(c2 * (1ll << (48 - s)) + (low >> s)),
+             (low & ((1ll << s) - 1)) == 0, s);
 }
 
 // round_div(2^48, d) for 1 <= d < 2^32: double estimate, exact correction.
@@ -632,8 +637,12 @@ __host__ __device__ __forceinline__ LnRow ln_row_consts(int sx, int sxx, int s, 
 //   inv = round_div(2^48, sd) from the reciprocal estimate after one Newton
 //     step: the floor is within one, and the exact remainder fixes it and
 //     decides the rounding;
-//   C = 2^47 - mean inv from 24-bit halves of mean and inv and 64-bit
-//     products with carries.
+//   -K_0 = floor((2^47 - mean inv) / 2^s): mean inv = p + pe exactly (fma),
+//     q = p 2^-s < 2^49 splits into its floor and a fraction fr (exact: its
+//     last bit is worth 2^-28 or more), and with |pe| 2^-s <= 2^-5 the
+//     remaining v = fr + pe 2^-s lies in (-1, 2), so floor(-v) is 0, -1 or -2
+//     by v > 0 and v > 1, two comparisons of exact values; 2^s divides C when
+//     v is 0 or 1.
 template <typename E>
 __host__ __device__ __forceinline__ LnRow ln_row_consts_e(int sx, int sxx, int s, int t) {
 #pragma clang fp contract(off)
@@ -667,16 +676,12 @@ __host__ __device__ __forceinline__ LnRow ln_row_consts_e(int sx, int sxx, int s
     rem -= sd;
   }
   if (2.0 * rem >= sd) inv += 1.0;
-  // C = 2^47 - mean inv with mean = m2 2^24 + m1, inv = i1 2^24 + i0
-  const double m2d = floor(mean * 0x1p-24), i1d = floor(inv * 0x1p-24);
-  const int m2 = (int)m2d, m1 = (int)fma(-m2d, 0x1p24, mean);
-  const int i1 = (int)i1d, i0 = (int)fma(-i1d, 0x1p24, inv);
-  const i64 p0 = (i64)((u64)(unsigned)m1 * (unsigned)i0);
-  const i64 p1 = (i64)m2 * i0 + (i64)m1 * i1;
-  const i64 p2 = (i64)m2 * i1;
-  const i64 t0 = (1ll << 47) - p0;
-  const i64 t1 = (t0 >> 24) - p1;
-  ln_row_fill(r, mean, inv, (t1 >> 24) - p2, ((t1 & 0xFFFFFF) << 24) | (t0 & 0xFFFFFF), s);
+  // -K_0 = floor(C / 2^s), C / 2^s = 2^(47-s) - q + ne
+  const double p = mean * inv, pe = fma(mean, inv, -p);
+  const double q = ldexp(p, -s), ne = -ldexp(pe, -s);
+  const double fq = floor(q), fr = q - fq, fr1 = fr - 1.0;
+  const double f = ((ldexp(1.0, 47 - s) - fq) - (fr > ne ? 1.0 : 0.0)) - (fr1 > ne ? 1.0 : 0.0);
+  ln_row_set(r, mean, inv, f, fr == ne || fr1 == ne, s);
   return r;
 }
 
@@ -752,6 +757,18 @@ __device__ __forceinline__ void ln32_elems(const int (&w)[NW], const int (&gm)[N
     out[q] = (int)pack_lo4(ov[4 * q], ov[4 * q + 1], ov[4 * q + 2], ov[4 * q + 3]);
 }
 
+// v summed over the LPR (8 or 16) lanes of its group, in every lane: DPP
+// moves, which stay off the LDS pipe a shuffle goes through.
+template <int LPR>
+__device__ __forceinline__ int group_sum(int v) {
+  static_assert(LPR == 8 || LPR == 16, "half or whole DPP rows");
+  v += __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false);   // lane ^ 1
+  v += __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false);   // lane ^ 2
+  v += __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false);  // mirrored half row
+  if (LPR == 16) v += __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false);  // mirrored row
+  return v;
+}
+
 template <int LPR>
 __device__ __forceinline__ bool ln32_row(const int (&w)[48 / LPR], const int (&gm)[48 / LPR],
                                          const int (&bt)[48 / LPR], const Ln32 &ln,
@@ -763,11 +780,8 @@ __device__ __forceinline__ bool ln32_row(const int (&w)[48 / LPR], const int (&g
     sx = __builtin_amdgcn_sdot4(w[q], 0x01010101, sx, false);
     sxx = __builtin_amdgcn_sdot4(w[q], w[q], sxx, false);
   }
-#pragma unroll
-  for (int off = 1; off < LPR; off <<= 1) {
-    sx += __shfl_xor(sx, off);
-    sxx += __shfl_xor(sxx, off);
-  }
+  sx = group_sum<LPR>(sx);
+  sxx = group_sum<LPR>(sxx);
   const LnRow r = ln_row_consts_e<LnEstHw>(sx, sxx, ln.s, ln.t);
   if (__any(r.tie))
     ln32_elems<true, NW>(w, gm, bt, ln, r, out);

@@ -899,12 +899,10 @@ __device__ __forceinline__ void ln_rows(const int8_t *src, int clamp, int8_t *ds
     }
   }
 #pragma unroll
-  for (int off = 1; off < 8; off <<= 1)
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      sx[r] += __shfl_xor(sx[r], off);
-      sxx[r] += __shfl_xor(sxx[r], off);
-    }
+  for (int r = 0; r < 2; ++r) {
+    sx[r] = group_sum<8>(sx[r]);
+    sxx[r] = group_sum<8>(sxx[r]);
+  }
   const int mr = sub & 1;
   LnRow mine = ln_row_consts_e<LnEstHw>(mr ? sx[1] : sx[0], mr ? sxx[1] : sxx[0], ln.s, ln.t);
   if (!two && mr) mine.tie = false;
@@ -1487,6 +1485,216 @@ __global__ __launch_bounds__(512, 4) void k_ffn32(GemmArgs g1, GemmArgs g2, LnPr
   }
 }
 
+// ---------------------------------------------------------------------------
+// The fused FFN over blocks of 16 rows by sixteen wavefronts (k_ffn16): the
+// phases of k_ffn32 for launches whose blocks fit one round of one per CU
+// (beyond it, a second round costs more than k_ffn32's larger blocks),
+// where the time is the chain of one block.  The MFMAs are 16x16x64: half a
+// packed weight tile (rows 16 hf .. +15 of the 32) against 16 token rows over
+// two K tiles, so a wavefront's share of each phase is a quarter to a half of
+// k_ffn32's:
+//   phase P  wavefront w < 12: projection columns 16 w .. (half w % 2 of
+//            packed tile w / 2), K = 192 in three steps;
+//   LN       16 lanes per row on wavefronts 0 .. 3, one per SIMD (on all
+//            sixteen the row constants, one chain per wavefront, would queue
+//            four deep on each SIMD);
+//   phase A  wavefront w: half tiles w, w + 16, w + 32 of FFN1's 48, their
+//            twelve lookups staged together;
+//   phase B  wavefront w < 12: FFN2 half tile w over K = 768, in two chains;
+//   LNE      as LN over the output rows.
+// Result lane l of a half tile holds token row l % 16, channels c .. c+3 with
+// c = 16 ((l / 16) % 2) + 8 hf + 4 (l / 32): one dword per tile.
+// Bound by that chain's latency.  One image (13 blocks), with the next
+// LayerNorm 1: 10.6 us, in k_ffn32's 7 blocks 13.4 us; the unpruned forward
+// of one image 290 -> 255 us, with the shorter LayerNorm constants.
+// ---------------------------------------------------------------------------
+static constexpr int kFfn16Rows = 16, kFfn16Waves = 16;
+
+// requant + align-add of four elements (the int32 form, or the exact one).
+__device__ __forceinline__ int res_quad(const GemmArgs &g, v4i acc, v4i bs, int r4, const Rq &ra,
+                                        const Rq &rb, int dirs, bool fast) {
+  int o[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r8 = __builtin_amdgcn_sbfe(r4, 8 * j, 8);
+    if (fast) {
+      const int t8 = dirs & 1 ? rq_dir_nowrap<true>(acc[j], ra) : rq_dir_nowrap<false>(acc[j], ra);
+      const int s = r8 * (1 << g.da) + t8 * (1 << g.db);
+      o[j] = dirs & 2 ? rq_dir<true>(s, rb) : rq_dir<false>(s, rb);
+    } else {
+      o[j] = epi_exact(EPI_RES, acc[j] - bs[j], bs[j], r8, g.shift_a, g.shift_b, g.da, g.db,
+                       g.os)[0];
+    }
+  }
+  return pack4(o[0], o[1], o[2], o[3]);
+}
+
+template <bool LNE>
+__global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, GemmArgs g2, Ln32 ln2,
+                                                               Ln32 lnn, GemmArgs gp, int dirsp,
+                                                               int dirs1, int dirs2) {
+  constexpr int NT = 64 * kFfn16Waves, ROW = kLnPrologueRow;
+  __shared__ __attribute__((aligned(16))) int8_t hid[kFfn16Rows * kFfnHRow];
+  __shared__ __attribute__((aligned(16))) int8_t rows_s[kFfn16Rows * ROW];  // y, LN2 rows; z
+  __shared__ __attribute__((aligned(16))) unsigned lut[kGeluLutMaxWords];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, grp = lane >> 4;
+  // this lane's 16 bytes of half tile t (16 output channels) at K step s
+  auto wfrag = [&](const int8_t *b, int kt_n, int t, int s) {
+    const int row = 16 * (t & 1) + l16 + 32 * (grp & 1);
+    return *reinterpret_cast<const v4i *>(
+        b + ((size_t)(t >> 1) * kt_n + 2 * s + (grp >> 1)) * 1024 + row * 16);
+  };
+  auto chan = [&](int t) { return 32 * (t >> 1) + 16 * (grp & 1) + 8 * (t & 1) + 4 * (grp >> 1); };
+  // loads that need no row index: the step table, the projection's and
+  // FFN1's weights and biases
+  static_assert(kGeluLutMaxWords / 4 <= 2 * NT, "one staging round");
+  const int n4 = g1.lut_words >> 2;
+  v4i tv[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    tv[i] = reinterpret_cast<const v4i *>(kGeluLut + g1.lut_off)[min(tid + NT * i, n4 - 1)];
+  const int wp = min(wave, 11);  // projection and FFN2 half tile (w < 12)
+  const int cp = chan(wp);
+  v4i pw[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s) pw[s] = wfrag(gp.b, 6, wp, s);
+  const v4i pbs = *reinterpret_cast<const v4i *>(gp.bias + cp);
+  const v4i bbs = *reinterpret_cast<const v4i *>(g2.bias + cp);
+  const int M = g1.m_dev ? min(*g1.m_dev, g1.m) : g1.m;
+  const int r0 = blockIdx.x * kFfn16Rows;
+  if (r0 >= M) return;  // uniform: before any barrier
+  const int arow = min(r0 + l16, M - 1);
+  v4i pa[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+    pa[s] = *reinterpret_cast<const v4i *>(gp.a + (size_t)arow * 192 + 64 * s + 16 * grp);
+  const int x4 = *reinterpret_cast<const int *>(gp.res + (size_t)arow * 192 + cp);
+  v4i w1[3][3], bs1[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    bs1[i] = *reinterpret_cast<const v4i *>(g1.bias + chan(wave + 16 * i));
+#pragma unroll
+    for (int s = 0; s < 3; ++s) w1[i][s] = wfrag(g1.b, 6, wave + 16 * i, s);
+  }
+  // LayerNorm parameters of this lane's 12 channels (wavefronts 0 .. 3)
+  const int sub = tid & 15, lrow = (tid >> 4) & 15;
+  int gm[3], bt[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    gm[q] = reinterpret_cast<const int *>(ln2.gamma + sub * 12)[q];
+    bt[q] = reinterpret_cast<const int *>(ln2.beta + sub * 12)[q];
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) reinterpret_cast<v4i *>(lut)[min(tid + NT * i, n4 - 1)] = tv[i];
+
+  auto fits = [&](const v4i &b, const GemmArgs &g) {
+    return tensor_narrow(g.bias_max, g.acc_lim) ||
+           __all(max(max(b[0], b[1]), max(b[2], b[3])) <= g.acc_lim &&
+                 min(min(b[0], b[1]), min(b[2], b[3])) >= -g.acc_lim);
+  };
+  // Phase P
+  int yres = 0;
+  if (wave < 12) {
+    const Rq rpa = rq_setup(gp.shift_a, -128, 127), rpb = rq_setup(gp.os, -128, 127);
+    v4i acc = pbs;
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(pw[s], pa[s], acc, 0, 0, 0);
+    yres = res_quad(gp, acc, pbs, x4, rpa, rpb, dirsp, fits(pbs, gp));
+    *reinterpret_cast<int *>(&rows_s[l16 * ROW + cp]) = yres;
+  }
+  __syncthreads();
+  // LayerNorm of rows_s by the first four wavefronts, in place or to out
+  auto norm = [&](const Ln32 &ln, int8_t *dst, int stride, int store_rows) {
+    int w[3], out[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) w[q] = reinterpret_cast<const int *>(&rows_s[lrow * ROW + sub * 12])[q];
+    ln32_row<16>(w, gm, bt, ln, out);  // (never a negative variance: ln_rows)
+    if (lrow < store_rows) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) reinterpret_cast<int *>(dst + lrow * stride + sub * 12)[q] = out[q];
+    }
+  };
+  if (wave < 4) norm(ln2, rows_s, ROW, kFfn16Rows);
+  __syncthreads();
+  // Phase A
+  {
+    v4i af[3], acc[3];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+      af[s] = *reinterpret_cast<const v4i *>(&rows_s[l16 * ROW + 64 * s + 16 * grp]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) acc[i] = bs1[i];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1[i][s], af[s], acc[i], 0, 0, 0);
+    const Rq r1a = rq_setup(g1.shift_a, -(1 << 23), (1 << 23) - 1);
+    int qhi = g1.lut_qhi;
+    asm("" : "+v"(qhi));
+    unsigned ov[3];
+    if (fits(bs1[0], g1) && fits(bs1[1], g1) && fits(bs1[2], g1)) {
+      int qv[12];
+      if (dirs1) {
+#pragma unroll
+        for (int j = 0; j < 12; ++j) qv[j] = shift_nowrap<true>(acc[j >> 2][j & 3], r1a);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 12; ++j) qv[j] = shift_nowrap<false>(acc[j >> 2][j & 3], r1a);
+      }
+      gelu_table_pack_n<12>(qv, ov, lut, g1.lut_cb, g1.lut_qlo, qhi);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        int o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          o[j] = epi_exact(EPI_GELU, acc[i][j] - bs1[i][j], bs1[i][j], 0, g1.shift_a, g1.shift_b,
+                           0, 0, 0)[0];
+        ov[i] = (unsigned)pack4(o[0], o[1], o[2], o[3]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      *reinterpret_cast<unsigned *>(&hid[l16 * kFfnHRow + chan(wave + 16 * i)]) = ov[i];
+  }
+  // Phase B: FFN2's weights load before the barrier
+  v4i w2[12];
+#pragma unroll
+  for (int s = 0; s < 12; ++s) w2[s] = wfrag(g2.b, 24, wp, s);
+  if (LNE) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      gm[q] = reinterpret_cast<const int *>(lnn.gamma + sub * 12)[q];
+      bt[q] = reinterpret_cast<const int *>(lnn.beta + sub * 12)[q];
+    }
+  }
+  __syncthreads();
+  if (wave < 12) {
+    const Rq r2a = rq_setup(g2.shift_a, -128, 127), r2b = rq_setup(g2.os, -128, 127);
+    v4i acc0 = bbs, acc1 = v4i{0};
+#pragma unroll
+    for (int s = 0; s < 12; s += 2) {
+      const int8_t *hp = &hid[l16 * kFfnHRow + 64 * s + 16 * grp];
+      acc0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2[s], *reinterpret_cast<const v4i *>(hp), acc0,
+                                                   0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+          w2[s + 1], *reinterpret_cast<const v4i *>(hp + 64), acc1, 0, 0, 0);
+    }
+    const int z4 = res_quad(g2, acc0 + acc1, bbs, yres, r2a, r2b, dirs2, fits(bbs, g2));
+    if (r0 + l16 < M)
+      *reinterpret_cast<int *>(reinterpret_cast<int8_t *>(g2.c) + (size_t)(r0 + l16) * 192 + cp) = z4;
+    if (LNE) *reinterpret_cast<int *>(&rows_s[l16 * ROW + cp]) = z4;
+  }
+  if constexpr (LNE) {
+    __syncthreads();
+    if (wave < 4) norm(lnn, lnn.out + (size_t)r0 * 192, 192, M - r0);
+  }
+}
+
 template <int DIRS1, bool LN, bool LNE, bool PJ>
 static void launch_ffn32_d(const GemmArgs &g1, const GemmArgs &g2, const LnPrologue &fl,
                            const LnPrologue &fe, const GemmArgs &gp, int dirsp, int dirs2,
@@ -1594,6 +1802,13 @@ int launch_ffn(const GemmArgs &g1_in, const GemmArgs &g2_in, hipStream_t s,
   const LnPrologue fl = ln ? *ln : LnPrologue{}, fe = ln_next ? *ln_next : LnPrologue{};
   const int dp = proj ? epilogue_dirs(gp, EPI_RES) : 0;
   const int mode = (ln ? 1 : 0) | (ln_next ? 2 : 0) | (d1 ? 4 : 0);
+  if (proj && rows == FFN_ROWS16) {
+    const dim3 grid16((g1.m + kFfn16Rows - 1) / kFfn16Rows), b16(64 * kFfn16Waves);
+    const Ln32 nn = ln_next ? ln_next->ln : Ln32{};
+    if (ln_next) hv_launch(k_ffn16<true>, grid16, b16, 0, s, g1, g2, ln->ln, nn, gp, dp, d1, d2);
+    else hv_launch(k_ffn16<false>, grid16, b16, 0, s, g1, g2, ln->ln, nn, gp, dp, d1, d2);
+    return check_hip(hipGetLastError(), "k_ffn16 launch");
+  }
   if (proj && rows32) {
     const dim3 grid32((g1.m + kFfn32Rows - 1) / kFfn32Rows);
     switch (mode) {

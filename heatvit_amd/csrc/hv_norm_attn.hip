@@ -164,12 +164,10 @@ __device__ __forceinline__ bool ln32_groups(const int8_t *__restrict__ x, const 
       }
     }
 #pragma unroll
-    for (int off = 1; off < 8; off <<= 1)
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        sx[r] += __shfl_xor(sx[r], off);
-        sxx[r] += __shfl_xor(sxx[r], off);
-      }
+    for (int r = 0; r < R; ++r) {
+      sx[r] = group_sum<8>(sx[r]);
+      sxx[r] = group_sum<8>(sxx[r]);
+    }
     // this lane's row of the R: sub % R
     int msx = sx[0], msxx = sxx[0];
 #pragma unroll
