@@ -125,26 +125,28 @@ __device__ __forceinline__ void state_invalid(int32_t *st) {
 // head statistics (3 -> 3), its PLAN layer (3 -> 3), and the weighted mean
 // of the head scores (plain mean, and the warning, when the weights sum to
 // zero).  The biases are any int32 and the reference adds them in int64
-// (gemm.py:118-119): the three products (|sum| < 2^16) are summed in 32
+// (gemm.py:118-119): the three products (|sum| < 2^16; weights and bias from LDS) are summed in 32
 // bits and the bias added in 64; the empty asm keeps the compiler from
 // folding bias and products into one 32-bit dot-product accumulation, which
 // wraps for biases near the int32 limits.
-__device__ __forceinline__ int fuse_hidden(const hv_selector_dev &p, const int8_t *stats, int j) {
+__device__ __forceinline__ int fuse_hidden(const hv_selector_dev &p, const int8_t *stats,
+                                           const int *wt, int bias) {
   const int a_in = -16 - (p.stats_out_exp + p.hw_w1_exp), a_out = p.hw_hidden_out_exp + 16;
   int dot = 0;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) dot += (int)stats[k] * (int)p.hw_w1t[j * 3 + k];
+  for (int k = 0; k < 3; ++k) dot += (int)stats[k] * wt[k];
   asm volatile("" : "+v"(dot));
-  return gelu_post((i64)p.hw_b1[j] + dot, a_in, a_out);
+  return gelu_post((i64)bias + dot, a_in, a_out);
 }
 
-__device__ __forceinline__ int fuse_weight(const hv_selector_dev &p, const int *hid, int j) {
+__device__ __forceinline__ int fuse_weight(const hv_selector_dev &p, const int *hid, const int *wt,
+                                           int bias) {
   const int b_sh = -16 - (p.hw_hidden_out_exp + p.hw_w2_exp);
   int dot = 0;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) dot += hid[k] * (int)p.hw_w2t[j * 3 + k];
+  for (int k = 0; k < 3; ++k) dot += hid[k] * wt[k];
   asm volatile("" : "+v"(dot));
-  return sat_q016(plan_sigmoid((int)requant_shift((i64)p.hw_b2[j] + dot, b_sh, 24)));
+  return sat_q016(plan_sigmoid((int)requant_shift((i64)bias + dot, b_sh, 24)));
 }
 
 // hs[0], hs[kMaxCand], hs[2 * kMaxCand]: the candidate's head scores; w[0..2]
@@ -172,10 +174,12 @@ __device__ __forceinline__ int fuse_mean(const int32_t *hs, const int *w, bool *
 // package_present, kept, pruned, warnings}; bad (any thread) marks the
 // image invalid (state token count -1).  Returns the kept count, or -1 when
 // the image is invalid; *den_out receives the sum of the partitioned
-// candidates' scores (the package's divisor).
+// candidates' scores (the package's divisor), thread 0's *warn_out the
+// image's warning bits.
 template <int NT>
 __device__ __forceinline__ int keep_list(int C, int pkg, int fc, bool warn, bool bad, int32_t *ki,
-                                         int32_t *st, i64 *den_out = nullptr) {
+                                         int32_t *st, i64 *den_out = nullptr,
+                                         int *warn_out = nullptr) {
   constexpr int NWAVE = NT / 64;
   __shared__ int w_kept[NWAVE], w_flags[NWAVE], w_den[NWAVE];
   const int c = threadIdx.x, lane = c & 63, wave = c >> 6;
@@ -222,6 +226,7 @@ __device__ __forceinline__ int keep_list(int C, int pkg, int fc, bool warn, bool
     const int warn_bits = ((any & 1) ? HV_WARN_HEAD_DEN_ZERO : 0) |
                           ((exists && den == 0) ? HV_WARN_PACKAGE_DEN_ZERO : 0);
     st[4] = warn_bits;
+    if (warn_out) *warn_out = warn_bits;
   }
   return kept;
 }
@@ -237,11 +242,14 @@ __device__ __forceinline__ int keep_list(int C, int pkg, int fc, bool warn, bool
 // ([G][192] ints) sums the groups.  Every thread of the NT-thread workgroup
 // calls it; cand points at candidate 0's row (16-byte aligned rows, RS
 // bytes apart, in memory or LDS).
-template <int NT, int RS, int G>
+template <int NT, int RS, int G, int Q>
 __device__ __forceinline__ void package_row(const int8_t *cand, int C, int pkg, int kept, int fv,
                                             i64 den, int8_t *dst, int *wgt, int *part_sum) {
   constexpr int kSteps = (kMaxCand + G - 1) / G;
-  static_assert(12 * G <= NT, "one thread per channel group and candidate group");
+  static_assert(12 * G <= NT && G % Q == 0 && 192 * Q <= NT, "one thread per sum");
+  // 208-word rows put a quad's four reads G / 4 rows apart (G = 36) on
+  // disjoint runs of 16 banks
+  constexpr int kPS = Q == 1 ? 192 : 208;
   const int tid = threadIdx.x;
   const int cg = tid / 12, chg = tid - cg * 12;
   v4i xv[kSteps];
@@ -264,43 +272,57 @@ __device__ __forceinline__ void package_row(const int8_t *cand, int C, int pkg, 
       const int c = cg + G * j;
       const int w = c < C ? wgt[c] : 0;
 #pragma unroll
-      for (int k = 0; k < 16; ++k) acc[k] += w * (int)(int8_t)(xv[j][k >> 2] >> (8 * (k & 3)));
+      for (int k = 0; k < 16; ++k)
+        acc[k] += __mul24(w, (int)(int8_t)(xv[j][k >> 2] >> (8 * (k & 3))));
     }
 #pragma unroll
-    for (int j = 0; j < 16; ++j) part_sum[cg * 192 + chg * 16 + j] = acc[j];
+    for (int j = 0; j < 16; ++j) part_sum[cg * kPS + chg * 16 + j] = acc[j];
   }
   __syncthreads();
   const int n_part = C - kept;
-  if (tid < 192) {
+  if (tid < 192 * Q) {
+    const int ch = tid / Q, g0 = tid % Q * (G / Q);
     int num = 0;
 #pragma unroll
-    for (int g = 0; g < G; ++g) num += part_sum[g * 192 + tid];
-    dst[tid] = (int8_t)sat_bits(round_div_pos_d(num, den == 0 ? n_part : den), 8);
+    for (int g = 0; g < G / Q; ++g) num += part_sum[(g0 + g) * kPS + ch];
+    if constexpr (Q == 4) {  // over the quad
+      num += __builtin_amdgcn_update_dpp(0, num, 0xB1, 0xf, 0xf, false);  // lane ^ 1
+      num += __builtin_amdgcn_update_dpp(0, num, 0x4E, 0xf, 0xf, false);  // lane ^ 2
+    }
+    dst[ch] = (int8_t)sat_bits(round_div_pos_d(num, den == 0 ? n_part : den), 8);
   }
 }
 
-// Eight GELU post-ops of a layer from its step table in LDS, packed four
+// N GELU post-ops of a layer from its step table in LDS, packed four
 // to a word: q = rsa(v, s) (or v << -s after the pre-clamp) with the
 // direction of the launch-uniform shift chosen once; the table's clamp
 // [qlo, qhi] lies inside the 24-bit range, so q needs no clamp of its own.
-__device__ __forceinline__ void sel_gelu_pack8(const int (&v)[8], const Rq &ra, const unsigned *lut,
-                                               const SelLut &t, unsigned (&ow)[2]) {
-  int q[8];
+template <int N>
+__device__ __forceinline__ void sel_gelu_pack(const int (&v)[N], const Rq &ra, const unsigned *lut,
+                                              const SelLut &t, unsigned (&ow)[N / 4]) {
+  int q[N];
   if (ra.s > 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) q[i] = (v[i] + ra.rnd + (v[i] >> 31)) >> ra.s;
+    for (int i = 0; i < N; ++i) q[i] = (v[i] + ra.rnd + (v[i] >> 31)) >> ra.s;
   } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) q[i] = min(max(v[i], ra.vlo), ra.vhi) << -ra.s;
+    for (int i = 0; i < N; ++i) q[i] = min(max(v[i], ra.vlo), ra.vhi) << -ra.s;
   }
-  gelu_table_pack_n<8>(q, ow, lut, t.cb, t.qlo, t.qhi);
+  gelu_table_pack_n<N>(q, ow, lut, t.cb, t.qlo, t.qhi);
+}
+
+// Orders this wavefront's LDS accesses before and after it as written (one
+// wavefront's LDS operations complete in order: no wait is needed).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 constexpr int kImgThreads = 1024, kXsRow = 208;
 
-// One workgroup per image (XCD-major).  Per layer, the (head, tile) units of
-// the three heads run over the eight wavefronts; the layer's GELU step table
-// (when its output shift has one) is staged once for the three heads:
+// One workgroup per image (XCD-major).  The three heads' (head, candidate
+// tile of 16) units run over the sixteen wavefronts, every unit's two column
+// tiles in one wavefront:
 //   local = GELU(x_h [C][64] . Wl [64][32] + bl)     16x16x64, 2 column tiles
 //   h1    = GELU(local . W1[0:32] + b1')             16x16x32, 2 column tiles
 //   h2    = GELU(h1 . W2 + b2)                       16x16x32, 1 column tile
@@ -308,30 +330,49 @@ constexpr int kImgThreads = 1024, kXsRow = 208;
 // every candidate, so the concat's second half is a per-head bias, exact in
 // 64 bits).  With the weights as the MFMA's first operand, result lane l of
 // a tile holds output channels 16 ct + 4 (l / 16) + i of candidate l % 16,
-// stored as one word.  Logits (16 -> 2), the 2-way softmax and the
-// lane mean of the head slice (the head statistic) are per candidate; the
+// stored as one word.  h1 and h2 of a unit depend only on its own local
+// rows, so both score layers run in one pass that rewrites the unit's rows
+// in place.  Logits (16 -> 2) and the 2-way softmax are per candidate; the
 // head fuse, the keep list and the package token follow in the same
 // workgroup.  The package row goes to pkg_rows[b] for k_selector_compact.
+//
+// Bound by the latency of its dependent phases (one workgroup per CU) and,
+// in the three GELU layers, by the CU's VALU issue.  So the unit index is
+// scalar, the biases start the accumulators, the head statistic is one MFMA
+// by ones, two step tables sit in LDS side by side, the head-weight layers
+// run in wavefronts that the global mean and fold leave idle, and constants
+// come from LDS, not memory, in the serial phases.  Over 64 sets of 197 tokens
+// 23.6 -> 19.2 us, 256 images 26.5 -> 20.3; of the earlier form's 22 us the
+// local layer took 5.8, score layer 1 4.3 and score layer 2 1.9 (units split
+// by column tile left every third round half empty), the head fuse 2.7 and the
+// package 1.8.
 __global__ __launch_bounds__(kImgThreads) void k_selector_image(
     hv_selector_dev p, const int8_t *tokens, const int32_t *offsets, int batch,
     const uint8_t *pkg_in, int fast_shifts, hv_selector_ckpt ck, SelLut tl, SelLut t1, SelLut t2,
     int32_t *fused_out, int32_t *kept_index, int32_t *state, int8_t *pkg_rows,
     int32_t *img_warn) {
-  constexpr int NT = kImgThreads;
-  __shared__ __attribute__((aligned(16))) unsigned lut[kGeluLutMaxWords];
+  constexpr int NT = kImgThreads, NW = NT / 64;
+  // step tables: [0, kGeluLutMaxWords) the local layer's, then score layer
+  // 2's; the second half score layer 1's; last the package sums
+  __shared__ __attribute__((aligned(16))) unsigned lut[2 * kGeluLutMaxWords];
+  unsigned *const lut_b = lut + kGeluLutMaxWords;
   __shared__ __attribute__((aligned(16))) int8_t wl[3][32 * 64];   // local_wt[h] [32][64]
   __shared__ __attribute__((aligned(16))) int8_t w1[3][32 * 64];   // w1t[h] [32][64]
   __shared__ __attribute__((aligned(16))) int8_t w2[3][16 * 32];   // w2t[h] [16][32]
   __shared__ int w3[3][8];                                         // w3t[h] [2][16] as words
-  __shared__ int bl[3][32], bb2[3][16];
-  __shared__ i64 bb1[3][32];                                       // b1 + global . W1[32:64]
-  // local [3][208][32], then h2 [3][208][16]; h1 [3][208][32]
-  __shared__ __attribute__((aligned(16))) int8_t act_a[3 * kCandPad * 32];
-  __shared__ __attribute__((aligned(16))) int8_t act_b[3 * kCandPad * 32];
+  __shared__ __attribute__((aligned(16))) int bl[3][32], bb2[3][16];
+  __shared__ int b1_s[3][32], b3_s[6];
+  __shared__ int hwc[24];  // hw_w1t [3][3], hw_w2t [3][3], hw_b1 [3], hw_b2 [3]
+  // b1 + global . W1[32:64]: its low 32 bits (exact where the int32 form runs) and in full
+  __shared__ __attribute__((aligned(16))) int bb1[3][32];
+  __shared__ i64 bbx[3][32];
+  // a unit's rows [candidate][32]: local, then h1, then h2 in the first 16 bytes
+  __shared__ __attribute__((aligned(16))) int8_t act[3 * kCandPad * 32];
   __shared__ int hs_s[3 * kMaxCand];                               // head scores [h][c]
   __shared__ int8_t st_s[kMaxCand * 3];                            // head statistics [c][h]
-  __shared__ int part[10][96];
-  __shared__ int glob_s[3][32];
+  __shared__ int hid_s[3 * kMaxCand], hw_s[3 * kMaxCand];          // head-weight MLP [c][j]
+  __shared__ unsigned part[5][24][2];
+  __shared__ __attribute__((aligned(16))) int8_t glob_s[3][32];
   __shared__ int fast_s[3][3];
   __shared__ int wgt[kMaxCand];
   // the image's candidate rows, 208-byte stride (conflict-free 16-byte
@@ -340,8 +381,8 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
 
   const int b = xcd_image(batch);
   if (b < 0) return;  // uniform: before any barrier
-  constexpr int NW = NT / 64;  // wavefronts; each takes two units per round, NW apart
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, grp = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row0 = offsets[b], N = offsets[b + 1] - row0, C = N - 1;
   const int pkg = pkg_in ? (pkg_in[b] ? 1 : 0) : 0;
   int32_t *st = state + (size_t)b * 5;
@@ -349,7 +390,7 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
     if (tid == 0) state_invalid(st);
     return;
   }
-  const int ntiles = (C + 15) >> 4;
+  const int ntiles = (C + 15) >> 4, nu = 3 * ntiles;
   const int8_t *cand = tokens + (size_t)(row0 + 1) * 192;
   // Candidate rows into LDS: every 16-byte load of the image in flight at
   // once (items past the end repeat the last one), stored after the weight
@@ -384,272 +425,215 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
     const u64 m = __ballot(fast_shifts && v <= lim32 && v >= -lim32);
     if ((tid & 15) == 0) fast_s[h][2] = ((unsigned)(m >> (16 * h)) & 0xFFFFu) == 0xFFFFu;
   }
+  if (tid >= 256 && tid < 352) b1_s[(tid - 256) >> 5][tid & 31] = p.b1[tid - 256];
+  if (tid >= 384 && tid < 390) b3_s[tid - 384] = p.b3[tid - 384];
+  if (tid >= 448 && tid < 472) {
+    const int i = tid - 448;
+    hwc[i] = i < 9 ? p.hw_w1t[i] : i < 18 ? p.hw_w2t[i - 9] : i < 21 ? p.hw_b1[i - 18]
+                                                                     : p.hw_b2[i - 21];
+  }
   if (tl.off >= 0) sel_stage_lut<NT>(tl, lut, tid);
 #pragma unroll
   for (int j = 0; j < kRowItems; ++j) {
     const int i = min(tid + j * NT, n_items - 1), c = i / 12;
     *reinterpret_cast<v4i *>(&xs[c * kXsRow + (i - c * 12) * 16]) = rv[j];
   }
-  // score layer 1's table loads in flight during the local layer
-  v4i lv[kLutRegs];
-  if (t1.off >= 0) lut_load<NT>(t1, lv, tid);
+  // the score layers' table loads in flight during the local layer
+  v4i lv1[kLutRegs], lv2[kLutRegs];
+  if (t1.off >= 0) lut_load<NT>(t1, lv1, tid);
+  if (t2.off >= 0) lut_load<NT>(t2, lv2, tid);
   __syncthreads();
 
-  // Local MLP and head statistics: unit u = h * nt2 + tile, tile = 2 rt + ct;
-  // two units per round, both candidate loads in flight, then their eight
-  // table lookups staged together.
+  // Local MLP and head statistics.
   {
     const int sh_in = -16 - (p.in_exp + p.local_w_exp), sh_out = p.local_out_exp + 16;
     const Rq ra = rq_setup(sh_in, -(1 << 23), (1 << 23) - 1), rb = rq_setup(sh_out, -128, 127);
-    // a second barrier here measured faster than none (three runs, about
-    // 1 us per launch)
-    __syncthreads();
-    const int nt2 = ntiles * 2, nu = 3 * nt2;
-    for (int u0 = wave; u0 < nu; u0 += 2 * NW) {
-      int hh[2], tv[2];
-      bool valid[2], fast[2];
-      v4i a[2], acc[2];
+    const v4i ones = v4i{0x01010101, 0x01010101, 0x01010101, 0x01010101};
+    for (int u = wave; u < nu; u += NW) {
+      const int h = (u >= ntiles ? 1 : 0) + (u >= 2 * ntiles ? 1 : 0);  // u / ntiles (< 3)
+      const int rt = u - h * ntiles, cc = rt * 16 + col;
+      const bool small = __builtin_amdgcn_readfirstlane(fast_s[h][0]) != 0;
+      const bool table = small && tl.off >= 0;
+      const v4i a =
+          *reinterpret_cast<const v4i *>(&xs[min(cc, C - 1) * kXsRow + h * 64 + grp * 16]);
+      v4i bias[2], acc[2];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int uu = min(u0 + NW * u, nu - 1);
-        valid[u] = u0 + NW * u < nu;
-        hh[u] = (uu >= nt2 ? 1 : 0) + (uu >= 2 * nt2 ? 1 : 0);  // uu / nt2 (< 3)
-        tv[u] = uu - hh[u] * nt2;
-        fast[u] = fast_s[hh[u]][0];
-        const int c = min((tv[u] >> 1) * 16 + col, C - 1);
-        a[u] = *reinterpret_cast<const v4i *>(&xs[c * kXsRow + hh[u] * 64 + grp * 16]);
+      for (int ct = 0; ct < 2; ++ct) {
+        bias[ct] = *reinterpret_cast<const v4i *>(&bl[h][ct * 16 + 4 * grp]);
+        const v4i wb = *reinterpret_cast<const v4i *>(&wl[h][(ct * 16 + col) * 64 + grp * 16]);
+        acc[ct] =
+            __builtin_amdgcn_mfma_i32_16x16x64_i8(wb, a, table ? bias[ct] : v4i{0}, 0, 0, 0);
       }
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const v4i wb =
-            *reinterpret_cast<const v4i *>(&wl[hh[u]][((tv[u] & 1) * 16 + col) * 64 + grp * 16]);
-        // weights as the first operand: lane (col, grp) gets output channels
-        // 16 ct + 4 grp + i of candidate 16 rt + col, stored as one word
-        acc[u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wb, a[u], v4i{0}, 0, 0, 0);
+      // lane mean of the candidate's 64 head lanes (selector.py:358-367):
+      // |sum| / 64 <= 128 needs no clamp below, and 127 * 64 none above
+      const int sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, a, v4i{0}, 0, 0, 0)[0];
+      if (grp == 0 && cc < C) {
+        const int8_t stat = (int8_t)((sum + 32 + (sum >> 31)) >> 6);
+        st_s[cc * 3 + h] = stat;
+        if (ck.head_stats) ck.head_stats[((size_t)b * kMaxCand + cc) * 3 + h] = stat;
       }
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int rt = tv[u] >> 1, cc = rt * 16 + col;
-        if (valid[u] && (tv[u] & 1) == 0) {
-          // lane mean of the candidate's 64 head lanes (selector.py:358-367)
-          int sum = 0;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) sum = dot4(a[u][k], 0x01010101, sum);
-          sum += __shfl_xor(sum, 16);
-          sum += __shfl_xor(sum, 32);
-          if (grp == 0 && cc < C) {
-            const int8_t stat = (int8_t)sat_bits(round_div_pos(sum, 64), 8);
-            st_s[cc * 3 + hh[u]] = stat;
-            if (ck.head_stats) ck.head_stats[((size_t)b * kMaxCand + cc) * 3 + hh[u]] = stat;
-          }
-        }
-      }
-      if (fast[0] && fast[1] && tl.off >= 0) {
-        int vv[8];
-        unsigned ow[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int jb = (tv[u] & 1) * 16 + 4 * grp;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) vv[4 * u + i] = acc[u][i] + bl[hh[u]][jb + i];
-        }
-        sel_gelu_pack8(vv, ra, lut, tl, ow);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int rt = tv[u] >> 1, jb = (tv[u] & 1) * 16 + 4 * grp;
-          if (valid[u])
-            *reinterpret_cast<unsigned *>(&act_a[(hh[u] * kCandPad + rt * 16 + col) * 32 + jb]) =
-                ow[u];
-        }
+      unsigned ow[2];
+      if (table) {
+        const int vv[8] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3],
+                           acc[1][0], acc[1][1], acc[1][2], acc[1][3]};
+        sel_gelu_pack<8>(vv, ra, lut, tl, ow);
       } else {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int rt = tv[u] >> 1, jb = (tv[u] & 1) * 16 + 4 * grp;
-          if (valid[u]) {
-            unsigned o[4];
+        for (int ct = 0; ct < 2; ++ct) {
+          unsigned o[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-              o[i] = (unsigned)(fast[u] && tl.off >= 0
-                                    ? (int)gelu_table_u8(rq(acc[u][i] + bl[hh[u]][jb + i], ra),
-                                                         lut, tl.cb, tl.qlo, tl.qhi)
-                                    : sel_gelu(acc[u][i], bl[hh[u]][jb + i], fast[u], ra, rb,
-                                               sh_in, sh_out));
-            *reinterpret_cast<unsigned *>(&act_a[(hh[u] * kCandPad + rt * 16 + col) * 32 + jb]) =
-                pack_lo4(o[0], o[1], o[2], o[3]);
-          }
+          for (int i = 0; i < 4; ++i)
+            o[i] = (unsigned)sel_gelu(acc[ct][i], bias[ct][i], small, ra, rb, sh_in, sh_out);
+          ow[ct] = pack_lo4(o[0], o[1], o[2], o[3]);
         }
       }
+      unsigned *dst = reinterpret_cast<unsigned *>(&act[(h * kCandPad + cc) * 32 + 4 * grp]);
+      dst[0] = ow[0];
+      dst[4] = ow[1];
     }
   }
+  if (t1.off >= 0) lut_store<NT>(t1, lv1, lut_b, tid);
   __syncthreads();
-  // score layer 1's table replaces the local layer's (barriers follow)
-  if (t1.off >= 0) lut_store<NT>(t1, lv, lut, tid);
-  // Global features = sat8(round_div(sum_c local, C)) per head and channel,
-  // five partial sums each; the local checkpoint before act_a is reused.
-  if (tid < 10 * 96) {
-    const int prt = tid / 96, hc = tid - prt * 96, h = hc >> 5, ch = hc & 31;
-    int sacc = 0;
-    for (int c = prt; c < C; c += 10) sacc += act_a[(h * kCandPad + c) * 32 + ch];
-    part[prt][hc] = sacc;
+  // score layer 2's table replaces the local layer's (barriers follow)
+  if (t2.off >= 0) lut_store<NT>(t2, lv2, lut, tid);
+  // Global features = sat8(round_div(sum_c local, C)) per head and channel:
+  // five wavefronts per head, one word of four channels per lane, summed as
+  // unsigned bytes (x + 128) in two 16-bit halves (196 * 255 < 2^16).
+  if (wave < 15) {
+    const int h = wave / 5, q = wave - 5 * h;
+    const unsigned *ap = reinterpret_cast<const unsigned *>(act + h * kCandPad * 32);
+    unsigned s0 = 0, s1 = 0;  // channels 4 w, 4 w + 2 and 4 w + 1, 4 w + 3
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const int c = 40 * k + 8 * q + (lane >> 3);  // < kCandPad
+      const unsigned x = c < C ? ap[c * 8 + (lane & 7)] ^ 0x80808080u : 0u;
+      s0 += x & 0x00FF00FFu;
+      s1 += (x >> 8) & 0x00FF00FFu;
+    }
+#pragma unroll
+    for (int off = 8; off <= 32; off <<= 1) {
+      s0 += __shfl_xor(s0, off);
+      s1 += __shfl_xor(s1, off);
+    }
+    if (lane < 8) {
+      part[q][h * 8 + lane][0] = s0;
+      part[q][h * 8 + lane][1] = s1;
+    }
   }
   if (ck.local)
     for (int i = tid; i < 3 * C * 2; i += NT) {
       const int h = i / (C * 2), k = i - h * C * 2;
       reinterpret_cast<v4i *>(ck.local + ((size_t)b * 3 + h) * kMaxCand * 32)[k] =
-          reinterpret_cast<const v4i *>(act_a + h * kCandPad * 32)[k];
+          reinterpret_cast<const v4i *>(act + h * kCandPad * 32)[k];
     }
   __syncthreads();
-  if (tid < 96) {
-    int sacc = 0;
+  if (wave < 3) {
+    // Wavefront h: head h's mean, then its fold into the bias.
+    const int h = wave;
+    if (lane < 32) {
+      unsigned s = 0;
 #pragma unroll
-    for (int q = 0; q < 10; ++q) sacc += part[q][tid];
-    const int gv = (int)sat_bits(round_div_pos_d(sacc, C), 8);
-    glob_s[tid >> 5][tid & 31] = gv;
-    if (ck.global) ck.global[((size_t)b * 3 + (tid >> 5)) * 32 + (tid & 31)] = (int8_t)gv;
+      for (int q = 0; q < 5; ++q) s += part[q][h * 8 + (lane >> 2)][lane & 1];
+      const int sacc = (int)((s >> (8 * (lane & 2))) & 0xFFFFu) - 128 * C;
+      const int gv = (int)sat_bits(round_div_pos_d(sacc, C), 8);
+      glob_s[h][lane] = (int8_t)gv;
+      if (ck.global) ck.global[((size_t)b * 3 + h) * 32 + lane] = (int8_t)gv;
+    }
+    wave_lds_fence();
+    if (lane < 32) {
+      // global . W1[32:64] in 32 bits (|sum| <= 32 * 128 * 127), the bias in 64
+      const int *wr = reinterpret_cast<const int *>(&w1[h][lane * 64 + 32]);
+      const int *gw = reinterpret_cast<const int *>(glob_s[h]);
+      int dot = 0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) dot = dot4(gw[q], wr[q], dot);
+      const i64 v = (i64)b1_s[h][lane] + dot;
+      bbx[h][lane] = v;
+      bb1[h][lane] = (int)v;
+      const u64 m = __ballot(fast_shifts && v <= lim32 && v >= -lim32);
+      if (lane == 0) fast_s[h][1] = (unsigned)m == 0xFFFFFFFFu;
+    }
+  } else {
+    // Head fuse, hidden layer: thread j * C + c of the other wavefronts takes
+    // head-weight unit j of candidate c.
+    const int i = tid - 192, j = (i >= C ? 1 : 0) + (i >= 2 * C ? 1 : 0), c = i - j * C;
+    static_assert(3 * kMaxCand <= NT - 192, "one thread per candidate and unit");
+    if (i < 3 * C) hid_s[c * 3 + j] = fuse_hidden(p, &st_s[c * 3], &hwc[3 * j], hwc[18 + j]);
   }
   __syncthreads();
-  if (tid < 96) {
-    // global . W1[32:64] in 32 bits (|sum| <= 32 * 128 * 127), the bias in 64
-    const int h = tid >> 5, j = tid & 31;
-    const int *wr = reinterpret_cast<const int *>(&w1[h][j * 64 + 32]);
-    int dot = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int gp = (glob_s[h][4 * q] & 0xFF) | ((glob_s[h][4 * q + 1] & 0xFF) << 8) |
-                     ((glob_s[h][4 * q + 2] & 0xFF) << 16) | (glob_s[h][4 * q + 3] << 24);
-      dot = dot4(gp, wr[q], dot);
-    }
-    const i64 v = (i64)p.b1[h * 32 + j] + dot;
-    bb1[h][j] = v;
-    const u64 m = __ballot(fast_shifts && v <= lim32 && v >= -lim32);
-    if (j == 0) fast_s[h][1] = (unsigned)(m >> (tid & 32)) == 0xFFFFFFFFu;
-  }
-  // Score layer 1 (local half): unit u = h * nt2 + 2 rt + ct, two units per
-  // round with their eight table lookups staged together.
+  // Head fuse, weight layer, over the last wavefronts (the first ones have a
+  // unit more below).
   {
-    const int sh_in = -16 - (p.concat_out_exp + p.score_w1_exp), sh_out = p.h1_out_exp + 16;
-    const Rq ra = rq_setup(sh_in, -(1 << 23), (1 << 23) - 1), rb = rq_setup(sh_out, -128, 127);
-    __syncthreads();
-    if (t2.off >= 0) lut_load<NT>(t2, lv, tid);  // score layer 2's table
-    const int nt2 = ntiles * 2, nu = 3 * nt2;
-    for (int u0 = wave; u0 < nu; u0 += 2 * NW) {
-      int hh[2], tv[2];
-      bool valid[2], fast[2];
+    const int i = NT - 1 - tid, j = (i >= C ? 1 : 0) + (i >= 2 * C ? 1 : 0), c = i - j * C;
+    if (i < 3 * C) {
+      const int w = fuse_weight(p, &hid_s[c * 3], &hwc[9 + 3 * j], hwc[21 + j]);
+      hw_s[c * 3 + j] = w;
+      if (ck.head_weights) ck.head_weights[((size_t)b * kMaxCand + c) * 3 + j] = w;
+    }
+  }
+  // Score layers 1 (local half) and 2 of each unit, in place.
+  {
+    const int sh1 = -16 - (p.concat_out_exp + p.score_w1_exp), so1 = p.h1_out_exp + 16;
+    const int sh2 = -16 - (p.h1_out_exp + p.score_w2_exp), so2 = p.h2_out_exp + 16;
+    const Rq ra1 = rq_setup(sh1, -(1 << 23), (1 << 23) - 1), rb1 = rq_setup(so1, -128, 127);
+    const Rq ra2 = rq_setup(sh2, -(1 << 23), (1 << 23) - 1), rb2 = rq_setup(so2, -128, 127);
+    for (int u = wave; u < nu; u += NW) {
+      const int h = (u >= ntiles ? 1 : 0) + (u >= 2 * ntiles ? 1 : 0);  // u / ntiles (< 3)
+      const int rt = u - h * ntiles;
+      int8_t *row = &act[(h * kCandPad + rt * 16 + col) * 32];
+      const bool small1 = __builtin_amdgcn_readfirstlane(fast_s[h][1]) != 0;
+      const bool small2 = __builtin_amdgcn_readfirstlane(fast_s[h][2]) != 0;
+      const bool table1 = small1 && t1.off >= 0, table2 = small2 && t2.off >= 0;
+      const long a = *reinterpret_cast<const long *>(row + grp * 8);
       v4i acc[2];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int uu = min(u0 + NW * u, nu - 1);
-        valid[u] = u0 + NW * u < nu;
-        hh[u] = (uu >= nt2 ? 1 : 0) + (uu >= 2 * nt2 ? 1 : 0);  // uu / nt2 (< 3)
-        tv[u] = uu - hh[u] * nt2;
-        fast[u] = fast_s[hh[u]][1];
-        const int rt = tv[u] >> 1, ct = tv[u] & 1;
-        const long a = *reinterpret_cast<const long *>(
-            &act_a[(hh[u] * kCandPad + rt * 16 + col) * 32 + grp * 8]);
+      for (int ct = 0; ct < 2; ++ct) {
         const long wb =
-            *reinterpret_cast<const long *>(&w1[hh[u]][(ct * 16 + col) * 64 + grp * 8]);
-        // weights first: four channels of one candidate per lane
-        acc[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, a, v4i{0}, 0, 0, 0);
+            *reinterpret_cast<const long *>(&w1[h][(ct * 16 + col) * 64 + grp * 8]);
+        const v4i bias = *reinterpret_cast<const v4i *>(&bb1[h][ct * 16 + 4 * grp]);
+        acc[ct] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, a, table1 ? bias : v4i{0}, 0, 0, 0);
       }
-      if (fast[0] && fast[1] && t1.off >= 0) {
-        int vv[8];
-        unsigned ow[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int jb = (tv[u] & 1) * 16 + 4 * grp;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) vv[4 * u + i] = acc[u][i] + (int)bb1[hh[u]][jb + i];
-        }
-        sel_gelu_pack8(vv, ra, lut, t1, ow);
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int jb = (tv[u] & 1) * 16 + 4 * grp;
-          if (valid[u])
-            *reinterpret_cast<unsigned *>(
-                &act_b[(hh[u] * kCandPad + (tv[u] >> 1) * 16 + col) * 32 + jb]) = ow[u];
-        }
+      unsigned ow[2];
+      if (table1) {
+        const int vv[8] = {acc[0][0], acc[0][1], acc[0][2], acc[0][3],
+                           acc[1][0], acc[1][1], acc[1][2], acc[1][3]};
+        sel_gelu_pack<8>(vv, ra1, lut_b, t1, ow);
       } else {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const int jb = (tv[u] & 1) * 16 + 4 * grp;
-          if (valid[u]) {
-            unsigned o[4];
+        for (int ct = 0; ct < 2; ++ct) {
+          unsigned o[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const i64 bias = bb1[hh[u]][jb + i];
-              o[i] = (unsigned)(fast[u] && t1.off >= 0
-                                    ? (int)gelu_table_u8(rq(acc[u][i] + (int)bias, ra), lut,
-                                                         t1.cb, t1.qlo, t1.qhi)
-                                : fast[u] ? rq(gelu_q16(rq(acc[u][i] + (int)bias, ra)), rb)
-                                          : gelu_exact64(acc[u][i], bias, sh_in, sh_out));
-            }
-            *reinterpret_cast<unsigned *>(
-                &act_b[(hh[u] * kCandPad + (tv[u] >> 1) * 16 + col) * 32 + jb]) =
-                pack_lo4(o[0], o[1], o[2], o[3]);
+          for (int i = 0; i < 4; ++i) {
+            const i64 bias = bbx[h][ct * 16 + 4 * grp + i];
+            o[i] = (unsigned)(small1 ? rq(gelu_q16(rq(acc[ct][i] + (int)bias, ra1)), rb1)
+                                     : gelu_exact64(acc[ct][i], bias, sh1, so1));
           }
+          ow[ct] = pack_lo4(o[0], o[1], o[2], o[3]);
         }
       }
-    }
-  }
-  __syncthreads();
-  if (t2.off >= 0) {  // score layer 2's table
-    lut_store<NT>(t2, lv, lut, tid);
-    __syncthreads();
-  }
-  // Score layer 2 into act_a ([3][208][16]): unit u = h * ntiles + rt, two
-  // units per round.
-  {
-    const int sh_in = -16 - (p.h1_out_exp + p.score_w2_exp), sh_out = p.h2_out_exp + 16;
-    const Rq ra = rq_setup(sh_in, -(1 << 23), (1 << 23) - 1), rb = rq_setup(sh_out, -128, 127);
-    const int nu = 3 * ntiles;
-    for (int u0 = wave; u0 < nu; u0 += 2 * NW) {
-      int hh[2], rt[2];
-      bool valid[2], fast[2];
-      v4i acc[2];
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int uu = min(u0 + NW * u, nu - 1);
-        valid[u] = u0 + NW * u < nu;
-        hh[u] = (uu >= ntiles ? 1 : 0) + (uu >= 2 * ntiles ? 1 : 0);  // uu / ntiles (< 3)
-        rt[u] = uu - hh[u] * ntiles;
-        fast[u] = fast_s[hh[u]][2];
-        const long a = *reinterpret_cast<const long *>(
-            &act_b[(hh[u] * kCandPad + rt[u] * 16 + col) * 32 + grp * 8]);
-        const long wb = *reinterpret_cast<const long *>(&w2[hh[u]][col * 32 + grp * 8]);
-        acc[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(wb, a, v4i{0}, 0, 0, 0);
-      }
-      if (fast[0] && fast[1] && t2.off >= 0) {
-        int vv[8];
-        unsigned ow[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) vv[4 * u + i] = acc[u][i] + bb2[hh[u]][4 * grp + i];
-        sel_gelu_pack8(vv, ra, lut, t2, ow);
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          if (valid[u])
-            *reinterpret_cast<unsigned *>(
-                &act_a[(hh[u] * kCandPad + rt[u] * 16 + col) * 16 + 4 * grp]) = ow[u];
+      wave_lds_fence();
+      unsigned *dst = reinterpret_cast<unsigned *>(row + 4 * grp);
+      dst[0] = ow[0];
+      dst[4] = ow[1];
+      wave_lds_fence();
+      const long a2 = *reinterpret_cast<const long *>(row + grp * 8);
+      const long wb2 = *reinterpret_cast<const long *>(&w2[h][col * 32 + grp * 8]);
+      const v4i bias2 = *reinterpret_cast<const v4i *>(&bb2[h][4 * grp]);
+      const v4i acc2 =
+          __builtin_amdgcn_mfma_i32_16x16x32_i8(wb2, a2, table2 ? bias2 : v4i{0}, 0, 0, 0);
+      unsigned o2[1];
+      if (table2) {
+        const int vv[4] = {acc2[0], acc2[1], acc2[2], acc2[3]};
+        sel_gelu_pack<4>(vv, ra2, lut, t2, o2);
       } else {
+        unsigned o[4];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          if (valid[u]) {
-            unsigned o[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int bias = bb2[hh[u]][4 * grp + i];
-              o[i] = (unsigned)(fast[u] && t2.off >= 0
-                                    ? (int)gelu_table_u8(rq(acc[u][i] + bias, ra), lut, t2.cb,
-                                                         t2.qlo, t2.qhi)
-                                    : sel_gelu(acc[u][i], bias, fast[u], ra, rb, sh_in, sh_out));
-            }
-            *reinterpret_cast<unsigned *>(
-                &act_a[(hh[u] * kCandPad + rt[u] * 16 + col) * 16 + 4 * grp]) =
-                pack_lo4(o[0], o[1], o[2], o[3]);
-          }
-        }
+        for (int i = 0; i < 4; ++i)
+          o[i] = (unsigned)sel_gelu(acc2[i], bias2[i], small2, ra2, rb2, sh2, so2);
+        o2[0] = pack_lo4(o[0], o[1], o[2], o[3]);
       }
+      wave_lds_fence();
+      dst[0] = o2[0];
     }
   }
   __syncthreads();
@@ -658,16 +642,20 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
     const int s3 = p.logits_out_exp - (p.h2_out_exp + p.score_w3_exp);
     const int sq = -16 - p.logits_out_exp;
     for (int i = tid; i < 3 * C; i += NT) {
-      const int h = i / C, c = i - h * C;
-      const v4i hv = *reinterpret_cast<const v4i *>(&act_a[(h * kCandPad + c) * 16]);
+      const int h = (i >= C ? 1 : 0) + (i >= 2 * C ? 1 : 0), c = i - h * C;
+      const v4i hv = *reinterpret_cast<const v4i *>(&act[(h * kCandPad + c) * 32]);
       int qv[2];
 #pragma unroll
       for (int lj = 0; lj < 2; ++lj) {
+        const int b3 = b3_s[h * 2 + lj];
         int acc = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) acc = dot4(hv[k], w3[h][lj * 4 + k], acc);
-        const int logit = (int)requant_shift((i64)acc + p.b3[h * 2 + lj], s3, 8);
-        qv[lj] = (int)requant_shift(logit, sq, 24);
+        // |acc| <= 16 * 2^14: the sum fits the int32 requant for |b3| <= 2^29
+        const int logit = b3 <= (1 << 29) && b3 >= -(1 << 29)
+                              ? requant_i32(acc + b3, s3, -128, 127)
+                              : (int)requant_shift((i64)acc + b3, s3, 8);
+        qv[lj] = requant_i32(logit, sq, -(1 << 23), (1 << 23) - 1);
       }
       const int mx = qv[0] > qv[1] ? qv[0] : qv[1];
       const unsigned e0 = softmax_exp(qv[0] - mx), e1 = softmax_exp(qv[1] - mx);
@@ -680,19 +668,7 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
     }
   }
   __syncthreads();
-  // Head fuse: thread j * C + c takes head-weight unit j of candidate c
-  // (hidden and weight layers, through LDS: the h1 buffer is free), then
-  // thread c < C the mean; keep list and state.
-  int *hid_s = reinterpret_cast<int *>(act_b), *hw_s = hid_s + 3 * kMaxCand;
-  const int fj = (tid >= C ? 1 : 0) + (tid >= 2 * C ? 1 : 0), fcand = tid - fj * C;
-  if (tid < 3 * C) hid_s[fcand * 3 + fj] = fuse_hidden(p, &st_s[fcand * 3], fj);
-  __syncthreads();
-  if (tid < 3 * C) {
-    const int w = fuse_weight(p, &hid_s[fcand * 3], fj);
-    hw_s[fcand * 3 + fj] = w;
-    if (ck.head_weights) ck.head_weights[((size_t)b * kMaxCand + fcand) * 3 + fj] = w;
-  }
-  __syncthreads();
+  // Head fuse, mean: thread c < C; keep list and state.
   int fc = 0;
   bool warn = false;
   if (tid < C) {
@@ -700,14 +676,15 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
     fused_out[(size_t)b * kMaxCand + tid] = fc;
   }
   i64 den = 0;
-  const int kept =
-      keep_list<NT>(C, pkg, fc, warn, false, kept_index + (size_t)b * kMaxCand, st, &den);
-  if (tid == 0 && img_warn) img_warn[b] |= st[4];
+  int warn_bits = 0;
+  const int kept = keep_list<NT>(C, pkg, fc, warn, false, kept_index + (size_t)b * kMaxCand, st,
+                                 &den, &warn_bits);
+  if (tid == 0 && img_warn && warn_bits) img_warn[b] |= warn_bits;
   if (kept < 0 || C - kept == 0) return;  // uniform; no package row
-  // (the step table's LDS is free: its last reader was score layer 2)
-  static_assert(36 * 192 <= kGeluLutMaxWords, "package sums fit the table's LDS");
-  package_row<NT, kXsRow, 36>(xs, C, pkg, kept, fc, den, pkg_rows + (size_t)b * 192, wgt,
-                              reinterpret_cast<int *>(lut));
+  // (the step tables' LDS is free: their last reader was score layer 2)
+  static_assert(36 * 208 <= 2 * kGeluLutMaxWords, "package sums fit the tables' LDS");
+  package_row<NT, kXsRow, 36, 4>(xs, C, pkg, kept, fc, den, pkg_rows + (size_t)b * 192, wgt,
+                                 reinterpret_cast<int *>(lut));
 }
 
 // finalize_tokens from given fused scores (hv_selector_finalize): the keep
@@ -810,7 +787,7 @@ __global__ __launch_bounds__(256) void k_selector_compact(
   if (lane == 0) red[wave] = d;
   __syncthreads();
   const i64 den = (i64)red[0] + red[1] + red[2] + red[3];
-  package_row<256, 192, 21>(tokens + (size_t)(row0 + 1) * 192, C, pkg, kept, fv, den, prow, wgt,
+  package_row<256, 192, 21, 1>(tokens + (size_t)(row0 + 1) * 192, C, pkg, kept, fv, den, prow, wgt,
                             part_sum);
 }
 

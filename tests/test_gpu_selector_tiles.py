@@ -1,0 +1,64 @@
+"""GPU selector at the edges of its 16-candidate tiles and of its per-head
+forms, against the CPU oracle, bit for bit: candidate counts around every
+multiple of the tile and of the wavefronts' rounds, with and without an
+incoming package; rows at the int8 limits (the global sums and the package
+sums at their largest); one head's biases beyond the int32 forms while the
+other heads stay within them; score layer 3 biases on both sides of the
+32-bit requant's bound."""
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+from heatvit_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ("local", "global_features", "head_scores", "head_stats", "head_weights", "fused_scores",
+        "tokens", "kept_index", "token_count", "warnings", "pruned_normal_count")
+
+
+def _check(oracle, sets, flags, params):
+    from heatvit_amd.selector import token_selector_batch
+    res = token_selector_batch(sets, flags, params)
+    for i, (t, f) in enumerate(zip(sets, flags)):
+        want = oracle.token_selector(t, f, params)
+        for k in KEYS:
+            assert np.array_equal(getattr(res[i], k), want[k]), (i, len(t) - 1, k)
+
+
+@pytest.mark.parametrize("candidates", (1, 2, 15, 16, 17, 31, 33, 79, 80, 81, 85, 86, 160, 161,
+                                        192, 193, 195, 196))
+def test_candidate_counts(oracle, candidates):
+    tokens, params = synth.selector_workload()
+    rng = np.random.default_rng(candidates)
+    random = rng.integers(-128, 128, (candidates + 1, 192)).astype(np.int8)
+    limits = rng.choice(np.array([-128, 127], np.int8), (candidates + 1, 192))
+    low = np.full((candidates + 1, 192), -128, np.int8)
+    sets = [tokens[0][:candidates + 1], random, limits, low]
+    flags = [False] * 4
+    if candidates > 1:
+        sets, flags = sets + sets[:3], flags + [True] * 3
+    _check(oracle, sets, flags, params)
+
+
+@pytest.mark.parametrize("head", (0, 1, 2))
+@pytest.mark.parametrize("part,name", (("local", "b"), ("score", "b1"), ("score", "b2")))
+def test_one_head_beyond_int32_forms(oracle, part, name, head):
+    tokens, params = synth.selector_workload()
+    sub = getattr(params, part)
+    bias = np.array(getattr(sub, name), np.int64)
+    bias[head, -1] = (1 << 31) - 1
+    bias[head, 0] = -(1 << 31)
+    params = dataclasses.replace(params, **{part: dataclasses.replace(sub, **{name: bias})})
+    _check(oracle, [tokens[0], tokens[1][:34]], [False, True], params)
+
+
+@pytest.mark.parametrize("bias", (1 << 29, (1 << 29) + 1))
+def test_score3_bias_bound(oracle, bias):
+    tokens, params = synth.selector_workload()
+    old = np.asarray(params.score.b3)
+    b3 = np.where(np.arange(old.size).reshape(old.shape) % 2, bias, -bias).astype(np.int64)
+    params = dataclasses.replace(params, score=dataclasses.replace(params.score, b3=b3))
+    _check(oracle, [tokens[0], tokens[1][:18]], [False, True], params)
