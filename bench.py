@@ -103,11 +103,13 @@ def class_work(counts, params, batch):
         hbm["ffn"] += (192 + 192 + 192 + (192 if chained else 0)) * t
         hbm["attention"] += (192 + 192) * t
         if stage_first:
-            hbm["layernorm"] += 2 * 192 * t
+            # after a selector the LayerNorm runs in its compaction: kept rows
+            # in, rows and LayerNorm out
+            hbm["layernorm"] += (2 if b == 1 else 3) * 192 * t
     for s in range(len(params.selectors)):
         c = counts[:, s] - 1
         ops["selector"] += int(2 * 13938 * c.sum())
-        hbm["selector"] += int((192 * counts[:, s] + 192 * counts[:, s + 1]).sum())
+        hbm["selector"] += int((192 * counts[:, s]).sum())
     ops["patch"] = 2 * 768 * 192 * 196 * batch
     hbm["patch"] = 150528 * batch + 197 * 192 * batch
     ops["head"] = 2 * 192 * 1000 * batch

@@ -50,11 +50,8 @@ static std::vector<ProfEvent> g_prof;
 // Active kernel class of the calling thread (-1: none).
 static thread_local int g_prof_cls = -1;
 
-struct ProfScope {
-  int prev;
-  ProfScope(int c, hipStream_t) : prev(g_prof_cls) { g_prof_cls = c; }
-  ~ProfScope() { g_prof_cls = prev; }
-};
+ProfScope::ProfScope(int c, hipStream_t) : prev(g_prof_cls) { g_prof_cls = c; }
+ProfScope::~ProfScope() { g_prof_cls = prev; }
 
 void prof_events(hipEvent_t *start, hipEvent_t *stop) {
   *start = *stop = nullptr;
@@ -769,6 +766,13 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
       a.fused = w.fused; a.kept_index = w.kept; a.state = st + (size_t)sel * batch * 5;
       a.pkg_rows = w.sel.pkg_rows;
       a.token_counts = token_counts; a.stage = sel + 1; a.img_warn = warnings;
+      // this block's LayerNorm 1 in the selector's compaction when it takes the
+      // int32 form (the rows, in w.xb, are 16-byte aligned)
+      const hv_block_dev &nb = p->blocks[blk - 1];
+      Ln32 ln;
+      if (ln32_setup(nb.ln1_gamma, nb.ln1_beta, w.blk.ln, nb.x_exp, nb.gamma1_exp, nb.beta1_exp,
+                     nb.ln1_out_exp, &ln))
+        a.ln = &ln;
       {
         ProfScope ps(HV_PROF_SELECTOR, s);
         rc = launch_selector(a, s);
@@ -777,6 +781,7 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
       std::swap(w.xa, w.xb);
       std::swap(w.off_a, w.off_b);
       std::swap(w.pkg_a, w.pkg_b);
+      if (a.ln) ln1_ready = w.blk.ln;
       ++sel;
       if (ckpt && (rc = launch_copy_ckpt(w.xa, w.off_a, batch, ckpt, ckpt_rows, sel, s))) return rc;
     }

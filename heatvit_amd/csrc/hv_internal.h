@@ -191,6 +191,13 @@ int launch_softmax_rows(const int32_t *x, const int32_t *offsets, int rows, uint
 int launch_primitive(int op, const int64_t *in, int64_t *out, int64_t n, int a, int b, int c,
                      hipStream_t s);
 
+// Profiler class of the launches in its scope (hv_profile_enable).
+struct ProfScope {
+  int prev;
+  ProfScope(int c, hipStream_t s);
+  ~ProfScope();
+};
+
 struct SelectorArgs {
   const hv_selector_dev *p;  // host copy passed by value; NULL: fused is an input
   const int8_t *tokens;
@@ -208,7 +215,22 @@ struct SelectorArgs {
   int stage;
   int32_t *img_warn;      // optional [B]: the state's warning bits are ORed in
   hv_selector_ckpt ck;    // optional intermediate outputs (null pointers skip)
+  const Ln32 *ln;         // optional (selector forward): also the LayerNorm of the output rows
 };
+// The selector forward's compaction (k_selector_rows); ln (optional): the
+// LayerNorm of the output rows too, into ln->out.
+struct SelectorRows {
+  const int8_t *tokens;
+  const int32_t *offsets, *kept_index, *state;
+  const int8_t *pkg_rows;
+  int8_t *out;
+  int32_t *out_offsets;
+  uint8_t *pkg_out;
+  int32_t *token_counts;  // optional [B][4] column `stage`
+  int32_t *img_warn;      // optional [B]
+  int batch, stage;
+};
+int launch_selector_rows(const SelectorRows &a, const Ln32 *ln, hipStream_t s);
 int launch_selector(const SelectorArgs &a, hipStream_t s);
 
 // Small utility kernels.

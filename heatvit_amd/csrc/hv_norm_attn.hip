@@ -233,6 +233,111 @@ __global__ __launch_bounds__(256) void k_layernorm32(const int8_t *__restrict__ 
   }
 }
 
+// Compaction of one selector's output (selector.py:456-500): workgroup (L, y)
+// takes output rows [32 y, 32 y + 32) of the image of logical index L
+// (XCD-major, as k_selector_image), eight lanes per row: CLS, the kept rows in
+// input order, then the package row, at the image's output offset (the token
+// counts of the images before it, an image with a bad count 0), and with LN
+// their LayerNorm 1 for the next block, from the registers that hold the row.
+// Each workgroup sums the counts before its image itself, one load per thread:
+// a separate one-workgroup scan over all counts cost a launch (4.5 us each on
+// the pruned batch-256 forward) against that sum.  Latency-bound (a chain of
+// two loads, the row sums and constants): one wavefront group per row instead
+// of one workgroup per image and a LayerNorm launch behind it, 256 images:
+// 5.4 + 5.9 -> 9.4 us at 88 tokens, 4.8 + 4.8 -> 5.5 at 30; 32 images 4.6 + 4.0
+// -> 5.0 and 4.1.
+template <bool LN>
+__global__ __launch_bounds__(256) void k_selector_rows(SelectorRows a, Ln32 ln) {
+  __shared__ int red[4];
+  const int B8 = (a.batch + 7) >> 3;
+  const int b = (blockIdx.x & 7) * B8 + (blockIdx.x >> 3);
+  if (b >= a.batch) return;
+  const int tid = threadIdx.x, sub = tid & 7, r = blockIdx.y * 32 + (tid >> 3);
+  const int32_t *st = a.state + (size_t)b * 5;
+  const int count = st[0], exists = st[1], kept = st[2];
+  // (-1, the list's padding, outside 1 <= r <= 196)
+  const int k = r >= 1 && r <= 196 ? a.kept_index[(size_t)b * 196 + r - 1] : -1;
+  const int row0 = a.offsets[b];
+  if (blockIdx.y > 0 && (int)blockIdx.y * 32 >= count) return;  // uniform
+  int sum = 0;
+  for (int i = tid; i < b; i += 256) sum += max(a.state[(size_t)i * 5], 0);
+  const bool live = r < count;
+  int w[6] = {0, 0, 0, 0, 0, 0};
+  if (live) {
+    const int8_t *src = r == 0      ? a.tokens + (size_t)row0 * 192
+                        : r <= kept ? a.tokens + (size_t)(row0 + 1 + k) * 192
+                                    : a.pkg_rows + (size_t)b * 192;
+    const int2 *xr = reinterpret_cast<const int2 *>(src + sub * 24);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int2 v = xr[q];
+      w[2 * q] = v.x;
+      w[2 * q + 1] = v.y;
+    }
+  }
+  int g[24], bb[24];
+  if constexpr (LN) {
+    const int2 *gp = reinterpret_cast<const int2 *>(ln.gamma + sub * 24);
+    const int2 *bp = reinterpret_cast<const int2 *>(ln.beta + sub * 24);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int2 gv = gp[q], bv = bp[q];
+      const int gw[2] = {gv.x, gv.y}, bw[2] = {bv.x, bv.y};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        g[8 * q + j] = __builtin_amdgcn_sbfe(gw[j >> 2], 8 * (j & 3), 8);
+        bb[8 * q + j] = __builtin_amdgcn_sbfe(bw[j >> 2], 8 * (j & 3), 8) * (1 << ln.bs);
+      }
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  if ((tid & 63) == 0) red[tid >> 6] = sum;
+  __syncthreads();
+  const int out0 = red[0] + red[1] + red[2] + red[3];
+  if (blockIdx.y == 0 && tid == 0) {
+    a.out_offsets[b] = out0;
+    if (b == a.batch - 1) a.out_offsets[a.batch] = out0 + max(count, 0);
+    a.pkg_out[b] = (uint8_t)(count > 0 ? exists : 0);
+    if (a.token_counts) a.token_counts[(size_t)b * 4 + a.stage] = count;
+  }
+  const size_t at = (size_t)(out0 + r) * 192 + sub * 24;
+  if (live) {
+    int2 *yr = reinterpret_cast<int2 *>(a.out + at);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) yr[q] = int2{w[2 * q], w[2 * q + 1]};
+  }
+  if constexpr (LN) {
+    int sx = 0, sxx = 0;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      sx = __builtin_amdgcn_sdot4(w[q], 0x01010101, sx, false);
+      sxx = __builtin_amdgcn_sdot4(w[q], w[q], sxx, false);
+    }
+    sx = group_sum<8>(sx);
+    sxx = group_sum<8>(sxx);
+    const LnRow c = ln_row_consts_e<LnEstHw>(sx, sxx, ln.s, ln.t);
+    if (live && c.neg_var && sub == 0 && a.img_warn)
+      atomicOr(&a.img_warn[b], HV_WARN_LN_NEGATIVE_VARIANCE);
+    const int rnd = 1 << (ln.os - 1);
+    int out[6];
+    if (__any(live && c.tie)) ln32_elems24<true>(w, g, bb, c, rnd, ln.os, out);
+    else ln32_elems24<false>(w, g, bb, c, rnd, ln.os, out);
+    if (live) {
+      int2 *yr = reinterpret_cast<int2 *>(ln.out + at);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) yr[q] = int2{out[2 * q], out[2 * q + 1]};
+    }
+  }
+}
+
+int launch_selector_rows(const SelectorRows &a, const Ln32 *ln, hipStream_t s) {
+  const dim3 grid((a.batch + 7) / 8 * 8, 7), block(256);  // 7 x 32 >= 197 rows
+  if (ln) hv_launch(k_selector_rows<true>, grid, block, 0, s, a, *ln);
+  else hv_launch(k_selector_rows<false>, grid, block, 0, s, a, Ln32{});
+  return check_hip(hipGetLastError(), "k_selector_rows launch");
+}
+
 // The int32 LayerNorm applies (and *ln is filled) when the input scale is in
 // [-16, -4], gamma sits at the common exponent, beta's shift is at most 22
 // and the output shift in [1, 29]; pointers must be 8-byte aligned.

@@ -14,10 +14,10 @@
 //   from memory by this workgroup only.
 // k_selector_keep (finalize_tokens from given fused scores): the keep list
 //   and state of one image per workgroup.
-// k_selector_compact, one workgroup per image with the same XCD-major
-//   order as k_selector_image: the image's output offset (the token counts
-//   of the images before it), then CLS, the kept rows in input order and
-//   the package row there (stream compaction).
+// k_selector_compact (the same): the image's output offset (the token counts
+//   of the images before it), then CLS, the kept rows in input order and the
+//   package row there (stream compaction).  k_selector_image's outputs take
+//   k_selector_rows, which can also write the rows' LayerNorm.
 //
 // GELU layers use the int32 requant/GELU path when the host finds every
 // shift in [-30, 30] and each layer's biases satisfy |b| <= 2^30 - 1 -
@@ -334,7 +334,7 @@ constexpr int kImgThreads = 1024, kXsRow = 208;
 // rows, so both score layers run in one pass that rewrites the unit's rows
 // in place.  Logits (16 -> 2) and the 2-way softmax are per candidate; the
 // head fuse, the keep list and the package token follow in the same
-// workgroup.  The package row goes to pkg_rows[b] for k_selector_compact.
+// workgroup.  The package row goes to pkg_rows[b] for k_selector_rows.
 //
 // Bound by the latency of its dependent phases (one workgroup per CU) and,
 // in the three GELU layers, by the CU's VALU issue.  So the unit index is
@@ -711,19 +711,14 @@ __global__ __launch_bounds__(256) void k_selector_keep(const int32_t *offsets,
   if (c == 0 && img_warn && st[0] > 0) img_warn[b] |= st[4];
 }
 
-// Stream compaction of one image (XCD-major, as k_selector_image): the
-// image's output offset (the token counts of the images before it; an image
-// with a bad count contributes 0), then CLS, the kept rows and the package
-// row there.  The package row comes from pkg_rows (selector forward) or is
-// computed here from the given fused scores (finalize).  Each workgroup
-// sums the counts before its image itself, one load per thread: a separate
-// one-workgroup scan kernel over all counts cost a launch (4.5 us each on
-// the pruned batch-256 forward) against that sum.
+// finalize_tokens' stream compaction of one image (XCD-major): the image's
+// output offset (the token counts of the images before it; an image with a
+// bad count contributes 0), then CLS, the kept rows and there the package row,
+// computed from the given fused scores.
 __global__ __launch_bounds__(256) void k_selector_compact(
     const int8_t *tokens, const int32_t *offsets, const uint8_t *pkg_in, int batch,
     const int32_t *fused, const int32_t *kept_index, const int32_t *state,
-    const int8_t *pkg_rows, int8_t *out, int32_t *out_offsets, uint8_t *pkg_out,
-    int32_t *token_counts, int stage) {
+    int8_t *out, int32_t *out_offsets, uint8_t *pkg_out, int32_t *token_counts, int stage) {
   __shared__ int wgt[kMaxCand];
   __shared__ int part_sum[21 * 192];
   __shared__ int src_k[kMaxCand + 1];
@@ -771,12 +766,6 @@ __global__ __launch_bounds__(256) void k_selector_compact(
   }
   if (!exists) return;
   int8_t *prow = out + (size_t)(out0 + 1 + kept) * 192;
-  if (pkg_rows) {
-    if (tid < 12)
-      reinterpret_cast<v4i *>(prow)[tid] =
-          reinterpret_cast<const v4i *>(pkg_rows + (size_t)b * 192)[tid];
-    return;
-  }
   // the partitioned candidates' score sum (finalize's scores are checked
   // to lie in [0, 65536], so a wavefront's sum fits 32 bits)
   const int fv = tid < C ? fused[(size_t)b * kMaxCand + tid] : 0;
@@ -812,14 +801,19 @@ int launch_selector(const SelectorArgs &a, hipStream_t s) {
               a.pkg_in, fast, a.ck, table(p.local_out_exp + 16), table(p.h1_out_exp + 16),
               table(p.h2_out_exp + 16), a.fused, a.kept_index, a.state, a.pkg_rows, a.img_warn);
     if ((rc = check_hip(hipGetLastError(), "k_selector_image launch"))) return rc;
-  } else {
-    hv_launch(k_selector_keep, grid, dim3(256), 0, s, a.offsets, a.pkg_in, a.batch, a.fused,
-              a.kept_index, a.state, a.img_warn);
-    if ((rc = check_hip(hipGetLastError(), "k_selector_keep launch"))) return rc;
+    const SelectorRows rows{a.tokens, a.offsets, a.kept_index, a.state, a.pkg_rows,
+                            a.out_tokens, a.out_offsets, a.pkg_out, a.token_counts, a.img_warn,
+                            a.batch, a.stage};
+    if (!a.ln) return launch_selector_rows(rows, nullptr, s);
+    const ProfScope ps(HV_PROF_LAYERNORM, s);  // the launch it stands in for
+    return launch_selector_rows(rows, a.ln, s);
   }
+  hv_launch(k_selector_keep, grid, dim3(256), 0, s, a.offsets, a.pkg_in, a.batch, a.fused,
+            a.kept_index, a.state, a.img_warn);
+  if ((rc = check_hip(hipGetLastError(), "k_selector_keep launch"))) return rc;
   hv_launch(k_selector_compact, grid, dim3(256), 0, s, a.tokens, a.offsets, a.pkg_in, a.batch,
-            a.fused, a.kept_index, a.state, a.p ? a.pkg_rows : nullptr, a.out_tokens,
-            a.out_offsets, a.pkg_out, a.token_counts, a.stage);
+            a.fused, a.kept_index, a.state, a.out_tokens, a.out_offsets, a.pkg_out,
+            a.token_counts, a.stage);
   return check_hip(hipGetLastError(), "k_selector_compact launch");
 }
 

@@ -4,7 +4,8 @@ multiple of the tile and of the wavefronts' rounds, with and without an
 incoming package; rows at the int8 limits (the global sums and the package
 sums at their largest); one head's biases beyond the int32 forms while the
 other heads stay within them; score layer 3 biases on both sides of the
-32-bit requant's bound."""
+32-bit requant's bound; and the compaction that also writes the next block's
+LayerNorm 1, through the model at batches around its groups of eight."""
 
 import dataclasses
 
@@ -62,3 +63,14 @@ def test_score3_bias_bound(oracle, bias):
     b3 = np.where(np.arange(old.size).reshape(old.shape) % 2, bias, -bias).astype(np.int64)
     params = dataclasses.replace(params, score=dataclasses.replace(params.score, b3=b3))
     _check(oracle, [tokens[0], tokens[1][:18]], [False, True], params)
+
+
+@pytest.mark.parametrize("batch", (1, 7, 8, 9, 17))
+def test_model_compaction_with_layernorm(oracle, batch):
+    from heatvit_amd.model import HeatViTModel
+    images, params = synth.pruned_workload(batch)
+    got = HeatViTModel().infer_batch(images, params)
+    logits, counts, _, warnings = oracle.model_infer_batch(images, params, threads=4)
+    assert np.array_equal(got.logits, logits)
+    assert np.array_equal(got.token_counts, counts)
+    assert np.array_equal(got.warnings, warnings)
