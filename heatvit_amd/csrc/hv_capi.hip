@@ -77,77 +77,6 @@ static void prof_clear() {
 
 // ---------------------------------------------------------------- utilities
 
-// cls (optional): row 0 of each image's 197 rows in x is the CLS row,
-// align_add(cls, pos[0]) (transformer.py:130-145), written here rather than
-// by a launch of its own after the patch embedding.
-// The model's GEMM bias tensors whose largest |bias| the first kernel of a
-// forward writes (GemmArgs::bias_max): entry 4 * block + t for t = 0 bqkv,
-// 1 bproj, 2 b1, 3 b2.
-struct BiasJobs {
-  const int32_t *p[48];
-  unsigned *out;
-};
-__device__ constexpr int kBiasCount[4] = {576, 192, 768, 192};
-
-__global__ void k_init_offsets(int32_t *offsets, uint8_t *pkg, int32_t *token_counts,
-                               int32_t *warnings, int batch, int rows, hv_patch_dev cls,
-                               int8_t *x, BiasJobs bj, int init_blocks) {
-  if ((int)blockIdx.x >= init_blocks) {  // uniform: one bias tensor per workgroup
-    __shared__ unsigned red[4];
-    const int j = blockIdx.x - init_blocks, n = kBiasCount[j & 3];
-    unsigned m = 0;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-      const int b = bj.p[j][k];
-      m = max(m, b < 0 ? 0u - (unsigned)b : (unsigned)b);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) bj.out[j] = max(max(red[0], red[1]), max(red[2], red[3]));
-    return;
-  }
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i <= batch) offsets[i] = i * rows;
-  if (i < batch) {
-    pkg[i] = 0;
-    if (token_counts)
-      for (int s = 0; s < 4; ++s) token_counts[(size_t)i * 4 + s] = rows;
-    if (warnings) warnings[i] = 0;
-  }
-  if (x)
-    for (int j = i; j < batch * 192; j += gridDim.x * blockDim.x) {
-      const int b = j / 192, c = j - b * 192;
-      x[(size_t)b * HV_MAX_TOKENS * 192 + c] =
-          (int8_t)align_add_i8(cls.cls[c], cls.cls_exp, cls.pos[c], cls.pos_exp, cls.tokens_exp);
-    }
-}
-
-int launch_init_offsets(int32_t *offsets, uint8_t *pkg, int32_t *token_counts,
-                        int32_t *warnings, int batch, int rows, hipStream_t s,
-                        const hv_patch_dev *cls, int8_t *x, const hv_block_dev *blocks,
-                        unsigned *bias_max) {
-  // batch + 1 offsets; with the CLS rows, batch * 192 bytes (a superset);
-  // with blocks, 48 more workgroups for the bias bounds
-  const int items = cls && x ? batch * 192 : batch + 1;
-  const int init_blocks = (items + 255) / 256;
-  BiasJobs bj{};
-  const bool bias = blocks && bias_max;
-  if (bias) {
-    for (int i = 0; i < 12; ++i) {
-      bj.p[4 * i] = blocks[i].bqkv;
-      bj.p[4 * i + 1] = blocks[i].bproj;
-      bj.p[4 * i + 2] = blocks[i].b1;
-      bj.p[4 * i + 3] = blocks[i].b2;
-    }
-    bj.out = bias_max;
-  }
-  hv_launch(k_init_offsets, dim3(init_blocks + (bias ? 48 : 0)), dim3(256), 0, s, offsets, pkg,
-            token_counts, warnings, batch, rows, cls ? *cls : hv_patch_dev{}, cls ? x : nullptr,
-            bj, init_blocks);
-  return check_hip(hipGetLastError(), "k_init_offsets launch");
-}
-
 // The attention's skip condition (k_attention), reported per image.
 __global__ void k_image_check(const int32_t *offsets, int batch, int capacity, int32_t *status,
                               int32_t *warnings) {
@@ -669,7 +598,7 @@ struct ModelWs {
   BlockWs blk;
   int32_t *off_a, *off_b, *fused, *kept, *state;
   uint8_t *pkg_a, *pkg_b;
-  unsigned *bias_max;  // [12][4], k_init_offsets
+  unsigned *bias_max;  // [12][4], k_patch_init
   SelectorWs sel;
 };
 
@@ -723,12 +652,16 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
   int32_t *st = state ? state : w.state;
   int rc;
 
-  {
-    ProfScope ps(HV_PROF_OTHER, s);
-    rc = launch_init_offsets(w.off_a, w.pkg_a, token_counts, warnings, batch, HV_MAX_TOKENS,
-                             s, &p->patch, w.xa, p->blocks, w.bias_max);
+  // the start of a forward in the patch embedding's launch
+  ModelInit init{};
+  init.offsets = w.off_a; init.pkg = w.pkg_a; init.token_counts = token_counts;
+  init.warnings = warnings; init.batch = batch; init.bias_max = w.bias_max;
+  for (int i = 0; i < 12; ++i) {
+    init.bias[4 * i] = p->blocks[i].bqkv;
+    init.bias[4 * i + 1] = p->blocks[i].bproj;
+    init.bias[4 * i + 2] = p->blocks[i].b1;
+    init.bias[4 * i + 3] = p->blocks[i].b2;
   }
-  if (rc) return rc;
   {
     ProfScope ps(HV_PROF_PATCH, s);
     if (float_images) {
@@ -736,10 +669,10 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
       rc = launch_image_front(static_cast<const float *>(images), batch, p->patch.image_exp,
                               w.blk.hidden, true, s);
       if (rc == HV_OK)
-        rc = launch_patch_embed(p->patch, w.blk.hidden, batch, w.xa, s, true, false);
+        rc = launch_patch_embed(p->patch, w.blk.hidden, batch, w.xa, s, true, &init);
     } else {
       rc = launch_patch_embed(p->patch, static_cast<const int8_t *>(images), batch, w.xa, s,
-                              false, false);
+                              false, &init);
     }
   }
   if (rc) return rc;

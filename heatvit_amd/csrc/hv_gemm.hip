@@ -44,6 +44,8 @@
 // v << k stays inside int32); the other cases call the exact 64/128-bit
 // form, kept out of line.
 #include <atomic>
+#include <algorithm>
+
 #include "hv_device.h"
 #include "hv_internal.h"
 #include "gelu_lut.inc"  // generated at build time by gen_gelu_lut.py
@@ -468,8 +470,9 @@ __global__ __launch_bounds__(256) void k_gemm(GemmArgs g, int n_blocks) {
 // (conflict-free fragment reads).  The next chunk -- or the next tile's
 // first chunk -- and its weight fragments are loaded while the current
 // chunk's MFMAs run; one barrier per chunk.
+// Workgroup bid of nblk (a multiple of 8).
 template <int MT, int NT, int WM, int EPI, int AMODE, int KTC, bool FAST, int DIRS>
-__global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g, int n_blocks) {
+__device__ __forceinline__ void gemm_lds(const GemmArgs &g, int n_blocks, int bid, int nblk) {
   constexpr int WN = 4 / WM, BM = 32 * MT * WM, BT = NT * WN;
   constexpr int KC = 6, NCH = KTC / KC, ROW = 208;
   constexpr int PIECES = BM * 12, PPT = PIECES / 256;
@@ -492,7 +495,7 @@ __global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g, int n_blocks) {
   // first out-of-range tile ends the sequence.
   auto logical = [&](int t) { return t < 8 * T8 ? (t & 7) * T8 + (t >> 3) : T; };
 
-  int t = blockIdx.x;
+  int t = bid;
   int L = logical(t);
   if (L >= T) return;
 
@@ -557,7 +560,7 @@ __global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g, int n_blocks) {
       __syncthreads();
       // Next step: the following chunk of this tile or the next tile's first.
       if (c == NCH - 1) {
-        Ln = logical(t + (int)gridDim.x);
+        Ln = logical(t + nblk);
         more = Ln < T;
         if (more) load_step(Ln, 0);
       } else {
@@ -580,11 +583,66 @@ __global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g, int n_blocks) {
     epi_tile<MT, NT, EPI, FAST, DIRS>(g, acc, bias4, res4, r0, ct0, M, h, l32, rq_a, rq_b,
                                       nullptr);
     if (!more) break;
-    t += gridDim.x;
+    t += nblk;
     L = Ln;
     tile_rows(L, arow, r0, ct0);
     epi_operands<MT, NT, EPI>(g, arow, ct0, h, bias4, res4);
   }
+}
+
+template <int MT, int NT, int WM, int EPI, int AMODE, int KTC, bool FAST, int DIRS>
+__global__ __launch_bounds__(256) void k_gemm_lds(GemmArgs g, int n_blocks) {
+  gemm_lds<MT, NT, WM, EPI, AMODE, KTC, FAST, DIRS>(g, n_blocks, blockIdx.x, gridDim.x);
+}
+
+// The patch embedding of a forward: workgroups below gemm_blocks run the
+// GEMM, the others (running beside them) write what the rest of the forward
+// starts from (ModelInit) and the CLS rows: align_add(cls, pos[0])
+// (transformer.py:127-145).  As a launch of its own in front of the GEMM that
+// was 3.0 to 4.9 us at 1 to 256 images: both 11.8 -> 10.2 us at one image,
+// 12.6 -> 10.0 at 32, 26.2 -> 22.4 at 256.
+__device__ constexpr int kBiasCount[4] = {576, 192, 768, 192};
+
+__device__ __forceinline__ void model_init(const ModelInit &in, const hv_patch_dev &p, int8_t *x,
+                                           int bid) {
+  if (bid < 48) {  // uniform: one bias tensor per workgroup
+    __shared__ unsigned red[4];
+    const int n = kBiasCount[bid & 3];
+    unsigned m = 0;
+    for (int k = threadIdx.x; k < n; k += 256) {
+      const int b = in.bias[bid][k];
+      m = max(m, b < 0 ? 0u - (unsigned)b : (unsigned)b);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) in.bias_max[bid] = max(max(red[0], red[1]), max(red[2], red[3]));
+    return;
+  }
+  const int i = (bid - 48) * 256 + threadIdx.x;  // up to batch * 192, past batch + 1
+  if (i <= in.batch) in.offsets[i] = i * HV_MAX_TOKENS;
+  if (i < in.batch) {
+    in.pkg[i] = 0;
+    if (in.token_counts)
+      for (int s = 0; s < 4; ++s) in.token_counts[(size_t)i * 4 + s] = HV_MAX_TOKENS;
+    if (in.warnings) in.warnings[i] = 0;
+  }
+  if (i < in.batch * 192) {
+    const int b = i / 192, c = i - b * 192;
+    x[(size_t)b * HV_MAX_TOKENS * 192 + c] =
+        (int8_t)align_add_i8(p.cls[c], p.cls_exp, p.pos[c], p.pos_exp, p.tokens_exp);
+  }
+}
+
+template <int AMODE, bool FAST, int DIRS>
+__global__ __launch_bounds__(256) void k_patch_init(GemmArgs g, int n_blocks, int gemm_blocks,
+                                                    ModelInit in, hv_patch_dev p) {
+  if ((int)blockIdx.x >= gemm_blocks) {
+    model_init(in, p, static_cast<int8_t *>(g.c), blockIdx.x - gemm_blocks);
+    return;
+  }
+  gemm_lds<2, 1, 2, EPI_PATCH, AMODE, 24, FAST, DIRS>(g, n_blocks, blockIdx.x, gemm_blocks);
 }
 
 // Host-side set-up of the epilogue preconditions.
@@ -1889,8 +1947,37 @@ __global__ void k_cls_rows(const int8_t *cls, const int8_t *pos, int8_t *x, int 
         (int8_t)align_add_i8(cls[c], cls_exp, pos[c], pos_exp, tokens_exp);
 }
 
+// launch_gemm's checks and set-up for the patch GEMM, its grid (run_lds) and
+// the workgroups of model_init behind it.
+template <int AMODE>
+static int launch_patch_init(GemmArgs g, const hv_patch_dev &p, const ModelInit &in,
+                             hipStream_t s) {
+  if ((uintptr_t)g.a & 15)
+    return fail(HV_EVALUE, HV_ERR_ADDRESS, "gemm: images must be 16-byte aligned");
+  if (g.bias && ((uintptr_t)g.bias & 15))
+    return fail(HV_EVALUE, HV_ERR_ADDRESS, "gemm: bias must be 16-byte aligned");
+  epilogue_limits_pub(g, EPI_PATCH);
+  g.vec_out = ((uintptr_t)g.c & 15) == 0;
+  g.vec_res = ((uintptr_t)g.pos & 15) == 0;
+  const int n_blocks = 3;  // 192 columns in tiles of 64
+  const long long tiles = (long long)((g.m + 127) / 128) * n_blocks;
+  const int gemm = (int)std::min<long long>((tiles + 7) / 8 * 8, kLdsGridCap);
+  const dim3 grid(gemm + 48 + (in.batch * 192 + 255) / 256), block(256);
+  if (!fast_epilogue(g, EPI_PATCH)) {
+    hv_launch((k_patch_init<AMODE, false, 0>), grid, block, 0, s, g, n_blocks, gemm, in, p);
+  } else {
+    switch (epilogue_dirs(g, EPI_PATCH)) {
+      case 0: hv_launch((k_patch_init<AMODE, true, 0>), grid, block, 0, s, g, n_blocks, gemm, in, p); break;
+      case 1: hv_launch((k_patch_init<AMODE, true, 1>), grid, block, 0, s, g, n_blocks, gemm, in, p); break;
+      case 2: hv_launch((k_patch_init<AMODE, true, 2>), grid, block, 0, s, g, n_blocks, gemm, in, p); break;
+      default: hv_launch((k_patch_init<AMODE, true, 3>), grid, block, 0, s, g, n_blocks, gemm, in, p); break;
+    }
+  }
+  return check_hip(hipGetLastError(), "k_patch_init launch");
+}
+
 int launch_patch_embed(const hv_patch_dev &p, const int8_t *images, int batch, int8_t *x,
-                       hipStream_t s, bool patch_rows, bool cls_rows) {
+                       hipStream_t s, bool patch_rows, const ModelInit *init) {
   if (batch <= 0) return HV_OK;
   GemmArgs g{};
   g.a = images;
@@ -1907,8 +1994,11 @@ int launch_patch_embed(const hv_patch_dev &p, const int8_t *images, int batch, i
   g.res_exp = p.pos_exp;
   g.out_exp = p.tokens_exp;
   g.lda = patch_rows ? 768 : 0;
-  int rc = launch_gemm(g, patch_rows ? A_ROWS : A_PATCH, EPI_PATCH, s);
-  if (rc || !cls_rows) return rc;
+  if (init)
+    return patch_rows ? launch_patch_init<A_ROWS>(g, p, *init, s)
+                      : launch_patch_init<A_PATCH>(g, p, *init, s);
+  const int rc = launch_gemm(g, patch_rows ? A_ROWS : A_PATCH, EPI_PATCH, s);
+  if (rc) return rc;
   hv_launch(k_cls_rows, dim3(batch), dim3(192), 0, s, p.cls, p.pos, x, p.cls_exp,
                      p.pos_exp, p.tokens_exp);
   return check_hip(hipGetLastError(), "k_cls_rows launch");

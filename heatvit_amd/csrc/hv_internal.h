@@ -118,9 +118,21 @@ int launch_gelu_post(bool table, const int64_t *in, int64_t *out, int64_t n, int
 // patches of NHWC 224x224x3 images (or, with patch_rows, the patch matrix
 // [B*196][768] itself), epilogue adds the position rows, and the CLS rows
 // are written by a second small kernel.
-// cls_rows false: the CLS rows are written elsewhere (launch_init_offsets).
+// init (optional): the same launch also writes the CLS rows and a forward's
+// start: offsets [batch + 1] of HV_MAX_TOKENS rows an image, cleared package
+// flags, token counts (optional, [batch][4]) and cleared warnings (optional),
+// and in bias_max[4 * block + t] the largest |bias| of each block's bqkv,
+// bproj, b1 and b2 (GemmArgs::bias_max).
+struct ModelInit {
+  int32_t *offsets;
+  uint8_t *pkg;
+  int32_t *token_counts, *warnings;
+  unsigned *bias_max;
+  const int32_t *bias[48];
+  int batch;
+};
 int launch_patch_embed(const hv_patch_dev &p, const int8_t *images, int batch, int8_t *x,
-                       hipStream_t s, bool patch_rows = false, bool cls_rows = true);
+                       hipStream_t s, bool patch_rows = false, const ModelInit *init = nullptr);
 
 // Image front end: float CHW [B][3][224][224] -> int8 at input_exp, as flat
 // NHWC images or (patch_rows) as the patch matrix [B*196][768].
@@ -234,14 +246,6 @@ int launch_selector_rows(const SelectorRows &a, const Ln32 *ln, hipStream_t s);
 int launch_selector(const SelectorArgs &a, hipStream_t s);
 
 // Small utility kernels.
-// cls, x (optional): also writes the CLS row (row 0 of each image's
-// HV_MAX_TOKENS rows) of the patch embedding into x.  blocks, bias_max
-// (optional): also writes the largest |bias| of each block's bqkv, bproj,
-// b1 and b2 to bias_max[4 * block + t] (GemmArgs::bias_max).
-int launch_init_offsets(int32_t *offsets, uint8_t *pkg, int32_t *token_counts,
-                        int32_t *warnings, int batch, int rows_per_image, hipStream_t s,
-                        const hv_patch_dev *cls = nullptr, int8_t *x = nullptr,
-                        const hv_block_dev *blocks = nullptr, unsigned *bias_max = nullptr);
 // Per-image token-count check of a caller's offsets: status[b] =
 // HV_ERR_TOKEN_COUNT unless 1 <= count <= 197 and the rows lie in
 // [0, capacity), else 0; warnings[b] = 0.  Either pointer may be NULL.
