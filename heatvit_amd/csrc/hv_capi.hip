@@ -159,11 +159,12 @@ struct LnChain {
 // finish sooner, one forward at a time).
 static bool small_rows(long long rows) { return rows < 2 * 256 * 64; }
 
-// Whether 16-row blocks of `rows` rows take one round of one per CU (the
-// model counts half the capacity once a selector has cut the rows: any choice
-// gives the same outputs, and 32 pruned images, 2,800 rows and fewer, run
-// 11.6 us a launch in them against 13.4).
-static bool few_rows(long long rows) { return rows <= 16ll * device_cus(); }
+// Whether k_ffn16's blocks of `rows` rows take one round of one per CU: of 16
+// rows, or, once a selector has left an unknown part of them live, of 16 or 32
+// by the live count (k_ffn16 has both measured).
+static bool few_rows(long long rows, bool pruned) {
+  return rows <= (pruned ? 32ll : 16ll) * device_cus();
+}
 
 // Images per batch from which hv_block_forward's attention kernel runs the
 // QKV GEMM (the model's does at every batch size).
@@ -461,9 +462,9 @@ int hv_block_forward(const hv_block_dev *p, const int8_t *x, const int32_t *offs
     return rc;
   return block_forward(*p, x, offsets, batch, max_rows, z, ck, warnings, w, (hipStream_t)stream,
                        LnChain{}, nullptr,
-                       few_rows(max_rows)     ? FFN_ROWS16
-                       : small_rows(max_rows) ? FFN_ROWS32
-                                              : FFN_ROWS64_BALANCED,
+                       few_rows(max_rows, false) ? FFN_ROWS16
+                       : small_rows(max_rows)    ? FFN_ROWS32
+                                                 : FFN_ROWS64_BALANCED,
                        check);
 }
 
@@ -731,7 +732,7 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
     // ones split where that evens out the CUs' work; pipelined callers,
     // whose other batches fill the CUs a launch leaves idle, keep 64.
     const int ffn_rows = (options & HV_FWD_PIPELINED)                   ? FFN_ROWS64
-                         : few_rows(sel > 0 ? max_rows / 2 : max_rows)  ? FFN_ROWS16
+                         : few_rows(max_rows, sel > 0)                  ? FFN_ROWS16
                          : (sel > 0 || small_rows((long long)max_rows)) ? FFN_ROWS32
                                                                         : FFN_ROWS64_BALANCED;
     if ((rc = block_forward(p->blocks[blk - 1], w.xa, w.off_a, batch, max_rows, w.xb, nullptr,

@@ -45,6 +45,7 @@
 // form, kept out of line.
 #include <atomic>
 #include <algorithm>
+#include <type_traits>
 
 #include "hv_device.h"
 #include "hv_internal.h"
@@ -1545,8 +1546,7 @@ __global__ __launch_bounds__(512, 4) void k_ffn32(GemmArgs g1, GemmArgs g2, LnPr
 
 // ---------------------------------------------------------------------------
 // The fused FFN over blocks of 16 rows by sixteen wavefronts (k_ffn16): the
-// phases of k_ffn32 for launches whose blocks fit one round of one per CU
-// (beyond it, a second round costs more than k_ffn32's larger blocks),
+// phases of k_ffn32 for launches whose blocks fit one round of one per CU,
 // where the time is the chain of one block.  The MFMAs are 16x16x64: half a
 // packed weight tile (rows 16 hf .. +15 of the 32) against 16 token rows over
 // two K tiles, so a wavefront's share of each phase is a quarter to a half of
@@ -1565,17 +1565,27 @@ __global__ __launch_bounds__(512, 4) void k_ffn32(GemmArgs g1, GemmArgs g2, LnPr
 // Bound by that chain's latency.  One image (13 blocks), with the next
 // LayerNorm 1: 10.6 us, in k_ffn32's 7 blocks 13.4 us; the unpruned forward
 // of one image 290 -> 255 us, with the shorter LayerNorm constants.
+//
+// TWO: for capacities above one 16-row block per CU, of which a selector may
+// leave few rows or all of them; only the device knows the live count M.  The
+// launch has one workgroup per CU (ceil(m / 32) at least), and each takes 16
+// rows while M <= rows1 = 16 gridDim.x, else 32: a second row tile against the
+// same weight fragments, phase A's two chains interleaved, LN on eight
+// wavefronts.  With selectors that keep everything, 32 images take 385 us a
+// forward (436 with a second round of 16-row blocks, 372 in k_ffn32), with
+// those of the seeded model, 2,800 rows and fewer, 312 (330 in k_ffn32).
 // ---------------------------------------------------------------------------
 static constexpr int kFfn16Rows = 16, kFfn16Waves = 16;
 
 // requant + align-add of four elements (the int32 form, or the exact one).
+template <bool FAST>
 __device__ __forceinline__ int res_quad(const GemmArgs &g, v4i acc, v4i bs, int r4, const Rq &ra,
-                                        const Rq &rb, int dirs, bool fast) {
+                                        const Rq &rb, int dirs) {
   int o[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r8 = __builtin_amdgcn_sbfe(r4, 8 * j, 8);
-    if (fast) {
+    if (FAST) {
       const int t8 = dirs & 1 ? rq_dir_nowrap<true>(acc[j], ra) : rq_dir_nowrap<false>(acc[j], ra);
       const int s = r8 * (1 << g.da) + t8 * (1 << g.db);
       o[j] = dirs & 2 ? rq_dir<true>(s, rb) : rq_dir<false>(s, rb);
@@ -1587,24 +1597,31 @@ __device__ __forceinline__ int res_quad(const GemmArgs &g, v4i acc, v4i bs, int 
   return pack4(o[0], o[1], o[2], o[3]);
 }
 
-template <bool LNE>
+// This lane's 16 bytes of packed half tile t (16 output channels) at K step s,
+// and the first of the four channels it holds of the half tile's result.
+__device__ __forceinline__ v4i ffn16_weights(const int8_t *b, int kt_n, int t, int s) {
+  const int lane = threadIdx.x & 63, grp = lane >> 4;
+  const int row = 16 * (t & 1) + (lane & 15) + 32 * (grp & 1);
+  return *reinterpret_cast<const v4i *>(
+      b + ((size_t)(t >> 1) * kt_n + 2 * s + (grp >> 1)) * 1024 + row * 16);
+}
+__device__ __forceinline__ int ffn16_channel(int t) {
+  const int grp = (threadIdx.x & 63) >> 4;
+  return 32 * (t >> 1) + 16 * (grp & 1) + 8 * (t & 1) + 4 * (grp >> 1);
+}
+
+template <bool LNE, bool TWO>
 __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, GemmArgs g2, Ln32 ln2,
                                                                Ln32 lnn, GemmArgs gp, int dirsp,
-                                                               int dirs1, int dirs2) {
+                                                               int dirs1, int dirs2, int rows1) {
   constexpr int NT = 64 * kFfn16Waves, ROW = kLnPrologueRow;
-  __shared__ __attribute__((aligned(16))) int8_t hid[kFfn16Rows * kFfnHRow];
-  __shared__ __attribute__((aligned(16))) int8_t rows_s[kFfn16Rows * ROW];  // y, LN2 rows; z
+  __shared__ __attribute__((aligned(16))) int8_t hid[(TWO ? 2 : 1) * kFfn16Rows * kFfnHRow];
+  // y, LN2 rows; z
+  __shared__ __attribute__((aligned(16))) int8_t rows_s[(TWO ? 2 : 1) * kFfn16Rows * ROW];
   __shared__ __attribute__((aligned(16))) unsigned lut[kGeluLutMaxWords];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, grp = lane >> 4;
-  // this lane's 16 bytes of half tile t (16 output channels) at K step s
-  auto wfrag = [&](const int8_t *b, int kt_n, int t, int s) {
-    const int row = 16 * (t & 1) + l16 + 32 * (grp & 1);
-    return *reinterpret_cast<const v4i *>(
-        b + ((size_t)(t >> 1) * kt_n + 2 * s + (grp >> 1)) * 1024 + row * 16);
-  };
-  auto chan = [&](int t) { return 32 * (t >> 1) + 16 * (grp & 1) + 8 * (t & 1) + 4 * (grp >> 1); };
   // loads that need no row index: the step table, the projection's and
   // FFN1's weights and biases
   static_assert(kGeluLutMaxWords / 4 <= 2 * NT, "one staging round");
@@ -1614,30 +1631,35 @@ __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, Gemm
   for (int i = 0; i < 2; ++i)
     tv[i] = reinterpret_cast<const v4i *>(kGeluLut + g1.lut_off)[min(tid + NT * i, n4 - 1)];
   const int wp = min(wave, 11);  // projection and FFN2 half tile (w < 12)
-  const int cp = chan(wp);
+  const int cp = ffn16_channel(wp);
   v4i pw[3];
 #pragma unroll
-  for (int s = 0; s < 3; ++s) pw[s] = wfrag(gp.b, 6, wp, s);
+  for (int s = 0; s < 3; ++s) pw[s] = ffn16_weights(gp.b, 6, wp, s);
   const v4i pbs = *reinterpret_cast<const v4i *>(gp.bias + cp);
-  const v4i bbs = *reinterpret_cast<const v4i *>(g2.bias + cp);
   const int M = g1.m_dev ? min(*g1.m_dev, g1.m) : g1.m;
-  const int r0 = blockIdx.x * kFfn16Rows;
+  // row tiles of 16 (uniform)
+  const int nt = TWO && M > rows1 ? 2 : 1;
+  const int r0 = blockIdx.x * kFfn16Rows * nt;
   if (r0 >= M) return;  // uniform: before any barrier
-  const int arow = min(r0 + l16, M - 1);
   v4i pa[3];
+  int x4;
+  auto load_rows = [&](int t) {
+    const int arow = min(r0 + 16 * t + l16, M - 1);
 #pragma unroll
-  for (int s = 0; s < 3; ++s)
-    pa[s] = *reinterpret_cast<const v4i *>(gp.a + (size_t)arow * 192 + 64 * s + 16 * grp);
-  const int x4 = *reinterpret_cast<const int *>(gp.res + (size_t)arow * 192 + cp);
+    for (int s = 0; s < 3; ++s)
+      pa[s] = *reinterpret_cast<const v4i *>(gp.a + (size_t)arow * 192 + 64 * s + 16 * grp);
+    x4 = *reinterpret_cast<const int *>(gp.res + (size_t)arow * 192 + cp);
+  };
+  load_rows(0);
   v4i w1[3][3], bs1[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    bs1[i] = *reinterpret_cast<const v4i *>(g1.bias + chan(wave + 16 * i));
+    bs1[i] = *reinterpret_cast<const v4i *>(g1.bias + ffn16_channel(wave + 16 * i));
 #pragma unroll
-    for (int s = 0; s < 3; ++s) w1[i][s] = wfrag(g1.b, 6, wave + 16 * i, s);
+    for (int s = 0; s < 3; ++s) w1[i][s] = ffn16_weights(g1.b, 6, wave + 16 * i, s);
   }
-  // LayerNorm parameters of this lane's 12 channels (wavefronts 0 .. 3)
-  const int sub = tid & 15, lrow = (tid >> 4) & 15;
+  // LayerNorm parameters of this lane's 12 channels (wavefronts 0 .. 4 nt - 1)
+  const int sub = tid & 15, lrow = tid >> 4;
   int gm[3], bt[3];
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
@@ -1653,18 +1675,26 @@ __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, Gemm
                  min(min(b[0], b[1]), min(b[2], b[3])) >= -g.acc_lim);
   };
   // Phase P
-  int yres = 0;
+  int yres[2] = {};
   if (wave < 12) {
     const Rq rpa = rq_setup(gp.shift_a, -128, 127), rpb = rq_setup(gp.os, -128, 127);
-    v4i acc = pbs;
+#pragma unroll 1
+    for (int t = 0;;) {
+      v4i acc = pbs;
 #pragma unroll
-    for (int s = 0; s < 3; ++s)
-      acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(pw[s], pa[s], acc, 0, 0, 0);
-    yres = res_quad(gp, acc, pbs, x4, rpa, rpb, dirsp, fits(pbs, gp));
-    *reinterpret_cast<int *>(&rows_s[l16 * ROW + cp]) = yres;
+      for (int s = 0; s < 3; ++s)
+        acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(pw[s], pa[s], acc, 0, 0, 0);
+      const int y4 = fits(pbs, gp) ? res_quad<true>(gp, acc, pbs, x4, rpa, rpb, dirsp)
+                                   : res_quad<false>(gp, acc, pbs, x4, rpa, rpb, dirsp);
+      *reinterpret_cast<int *>(&rows_s[(16 * t + l16) * ROW + cp]) = y4;
+      yres[0] = t == 0 ? y4 : yres[0];
+      yres[1] = y4;
+      if (++t == nt) break;
+      load_rows(t);
+    }
   }
   __syncthreads();
-  // LayerNorm of rows_s by the first four wavefronts, in place or to out
+  // LayerNorm of rows_s by the first 4 nt wavefronts, in place or to out
   auto norm = [&](const Ln32 &ln, int8_t *dst, int stride, int store_rows) {
     int w[3], out[3];
 #pragma unroll
@@ -1675,14 +1705,14 @@ __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, Gemm
       for (int q = 0; q < 3; ++q) reinterpret_cast<int *>(dst + lrow * stride + sub * 12)[q] = out[q];
     }
   };
-  if (wave < 4) norm(ln2, rows_s, ROW, kFfn16Rows);
+  if (wave < 4 * nt) norm(ln2, rows_s, ROW, kFfn16Rows * nt);
   __syncthreads();
   // Phase A
-  {
-    v4i af[3], acc[3];
+  auto ffn1 = [&](v4i (&acc)[3], int t) {
+    v4i af[3];
 #pragma unroll
     for (int s = 0; s < 3; ++s)
-      af[s] = *reinterpret_cast<const v4i *>(&rows_s[l16 * ROW + 64 * s + 16 * grp]);
+      af[s] = *reinterpret_cast<const v4i *>(&rows_s[(16 * t + l16) * ROW + 64 * s + 16 * grp]);
 #pragma unroll
     for (int i = 0; i < 3; ++i) acc[i] = bs1[i];
 #pragma unroll
@@ -1690,21 +1720,45 @@ __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, Gemm
 #pragma unroll
       for (int i = 0; i < 3; ++i)
         acc[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w1[i][s], af[s], acc[i], 0, 0, 0);
+  };
+  auto store_hid = [&](const unsigned (&ov)[3], int t) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      *reinterpret_cast<unsigned *>(
+          &hid[(16 * t + l16) * kFfnHRow + ffn16_channel(wave + 16 * i)]) = ov[i];
+  };
+  auto gelu_tiles = [&](auto tiles) {  // int32 form, the tiles' chains interleaved
+    constexpr int N = decltype(tiles)::value;
+    v4i acc[N][3];
+#pragma unroll
+    for (int t = 0; t < N; ++t) ffn1(acc[t], t);
     const Rq r1a = rq_setup(g1.shift_a, -(1 << 23), (1 << 23) - 1);
     int qhi = g1.lut_qhi;
     asm("" : "+v"(qhi));
-    unsigned ov[3];
-    if (fits(bs1[0], g1) && fits(bs1[1], g1) && fits(bs1[2], g1)) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
       int qv[12];
+      unsigned ov[3];
       if (dirs1) {
 #pragma unroll
-        for (int j = 0; j < 12; ++j) qv[j] = shift_nowrap<true>(acc[j >> 2][j & 3], r1a);
+        for (int j = 0; j < 12; ++j) qv[j] = shift_nowrap<true>(acc[t][j >> 2][j & 3], r1a);
       } else {
 #pragma unroll
-        for (int j = 0; j < 12; ++j) qv[j] = shift_nowrap<false>(acc[j >> 2][j & 3], r1a);
+        for (int j = 0; j < 12; ++j) qv[j] = shift_nowrap<false>(acc[t][j >> 2][j & 3], r1a);
       }
       gelu_table_pack_n<12>(qv, ov, lut, g1.lut_cb, g1.lut_qlo, qhi);
-    } else {
+      store_hid(ov, t);
+    }
+  };
+  if (fits(bs1[0], g1) && fits(bs1[1], g1) && fits(bs1[2], g1)) {
+    if (nt == 1) gelu_tiles(std::integral_constant<int, 1>());
+    else gelu_tiles(std::integral_constant<int, TWO ? 2 : 1>());
+  } else {
+#pragma unroll 1
+    for (int t = 0; t < nt; ++t) {
+      v4i acc[3];
+      unsigned ov[3];
+      ffn1(acc, t);
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         int o[4];
@@ -1714,15 +1768,14 @@ __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, Gemm
                            0, 0, 0)[0];
         ov[i] = (unsigned)pack4(o[0], o[1], o[2], o[3]);
       }
+      store_hid(ov, t);
     }
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-      *reinterpret_cast<unsigned *>(&hid[l16 * kFfnHRow + chan(wave + 16 * i)]) = ov[i];
   }
-  // Phase B: FFN2's weights load before the barrier
+  // Phase B: FFN2's weights and biases load before the barrier
   v4i w2[12];
 #pragma unroll
-  for (int s = 0; s < 12; ++s) w2[s] = wfrag(g2.b, 24, wp, s);
+  for (int s = 0; s < 12; ++s) w2[s] = ffn16_weights(g2.b, 24, wp, s);
+  const v4i bbs = *reinterpret_cast<const v4i *>(g2.bias + cp);
   if (LNE) {
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -1733,23 +1786,31 @@ __global__ __launch_bounds__(64 * kFfn16Waves, 4) void k_ffn16(GemmArgs g1, Gemm
   __syncthreads();
   if (wave < 12) {
     const Rq r2a = rq_setup(g2.shift_a, -128, 127), r2b = rq_setup(g2.os, -128, 127);
-    v4i acc0 = bbs, acc1 = v4i{0};
+#pragma unroll 1
+    for (int t = 0; t < nt; ++t) {
+      const int row = 16 * t + l16;
+      v4i acc0 = bbs, acc1 = v4i{0};
 #pragma unroll
-    for (int s = 0; s < 12; s += 2) {
-      const int8_t *hp = &hid[l16 * kFfnHRow + 64 * s + 16 * grp];
-      acc0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2[s], *reinterpret_cast<const v4i *>(hp), acc0,
-                                                   0, 0, 0);
-      acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(
-          w2[s + 1], *reinterpret_cast<const v4i *>(hp + 64), acc1, 0, 0, 0);
+      for (int s = 0; s < 12; s += 2) {
+        const int8_t *hp = &hid[row * kFfnHRow + 64 * s + 16 * grp];
+        acc0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(w2[s], *reinterpret_cast<const v4i *>(hp),
+                                                     acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+            w2[s + 1], *reinterpret_cast<const v4i *>(hp + 64), acc1, 0, 0, 0);
+      }
+      const v4i acc = acc0 + acc1;
+      const int z4 = fits(bbs, g2) ? res_quad<true>(g2, acc, bbs, yres[0], r2a, r2b, dirs2)
+                                   : res_quad<false>(g2, acc, bbs, yres[0], r2a, r2b, dirs2);
+      if (r0 + row < M)
+        *reinterpret_cast<int *>(reinterpret_cast<int8_t *>(g2.c) + (size_t)(r0 + row) * 192 + cp) =
+            z4;
+      if (LNE) *reinterpret_cast<int *>(&rows_s[row * ROW + cp]) = z4;
+      yres[0] = yres[1];
     }
-    const int z4 = res_quad(g2, acc0 + acc1, bbs, yres, r2a, r2b, dirs2, fits(bbs, g2));
-    if (r0 + l16 < M)
-      *reinterpret_cast<int *>(reinterpret_cast<int8_t *>(g2.c) + (size_t)(r0 + l16) * 192 + cp) = z4;
-    if (LNE) *reinterpret_cast<int *>(&rows_s[l16 * ROW + cp]) = z4;
   }
   if constexpr (LNE) {
     __syncthreads();
-    if (wave < 4) norm(lnn, lnn.out + (size_t)r0 * 192, 192, M - r0);
+    if (wave < 4 * nt) norm(lnn, lnn.out + (size_t)r0 * 192, 192, M - r0);
   }
 }
 
@@ -1861,10 +1922,20 @@ int launch_ffn(const GemmArgs &g1_in, const GemmArgs &g2_in, hipStream_t s,
   const int dp = proj ? epilogue_dirs(gp, EPI_RES) : 0;
   const int mode = (ln ? 1 : 0) | (ln_next ? 2 : 0) | (d1 ? 4 : 0);
   if (proj && rows == FFN_ROWS16) {
-    const dim3 grid16((g1.m + kFfn16Rows - 1) / kFfn16Rows), b16(64 * kFfn16Waves);
+    const int n16 = (g1.m + kFfn16Rows - 1) / kFfn16Rows, cus = device_cus();
+    const dim3 b16(64 * kFfn16Waves);
     const Ln32 nn = ln_next ? ln_next->ln : Ln32{};
-    if (ln_next) hv_launch(k_ffn16<true>, grid16, b16, 0, s, g1, g2, ln->ln, nn, gp, dp, d1, d2);
-    else hv_launch(k_ffn16<false>, grid16, b16, 0, s, g1, g2, ln->ln, nn, gp, dp, d1, d2);
+    auto go = [&](auto k, int blocks) {
+      hv_launch(k, dim3(blocks), b16, 0, s, g1, g2, ln->ln, nn, gp, dp, d1, d2, kFfn16Rows * blocks);
+    };
+    if (n16 <= cus) {
+      if (ln_next) go(k_ffn16<true, false>, n16);
+      else go(k_ffn16<false, false>, n16);
+    } else {  // workgroups of 32 rows cover the capacity in any case
+      const int blocks = std::max(cus, (n16 + 1) / 2);
+      if (ln_next) go(k_ffn16<true, true>, blocks);
+      else go(k_ffn16<false, true>, blocks);
+    }
     return check_hip(hipGetLastError(), "k_ffn16 launch");
   }
   if (proj && rows32) {

@@ -100,8 +100,9 @@ struct LnPrologue {
 //   FFN_ROWS64_BALANCED  k_ffn, with the last 64-row blocks split into
 //                        32-row ones when the blocks exceed a whole number
 //                        of blocks per CU by at most half the CUs.
-//   FFN_ROWS16           blocks of 16 rows by sixteen wavefronts (k_ffn16), for
-//                        launches of at most one such block per CU.
+//   FFN_ROWS16           blocks of 16 rows by sixteen wavefronts (k_ffn16), or of
+//                        32 where the live rows exceed one block of 16 per CU
+//                        (capacities up to 32 rows per CU).
 enum FfnRows { FFN_ROWS64 = 0, FFN_ROWS32 = 1, FFN_ROWS64_BALANCED = 2, FFN_ROWS16 = 3 };
 int launch_ffn(const GemmArgs &g1, const GemmArgs &g2, hipStream_t s,
                const LnPrologue *ln = nullptr, const LnPrologue *ln_next = nullptr,
