@@ -177,6 +177,7 @@ static constexpr int kFusedQkvMinBatch = 32;
 // ffn_rows: the fused FFN's row blocking (FfnRows, launch_ffn).
 // check: the per-image status and cleared warnings, written by the attention
 // kernel (hv_block_forward without a separate image check).
+// pipelined: HV_FWD_PIPELINED.
 struct ImageCheck {
   int32_t *status, *warnings;
 };
@@ -184,7 +185,8 @@ static int block_forward(const hv_block_dev &p, const int8_t *x, const int32_t *
                          int batch, int max_rows, int8_t *z, const hv_block_ckpt *ck,
                          int32_t *warnings, const BlockWs &w, hipStream_t s,
                          const LnChain &chain = LnChain{}, const unsigned *bias_max = nullptr,
-                         int ffn_rows = FFN_ROWS64, const ImageCheck &check = ImageCheck{}) {
+                         int ffn_rows = FFN_ROWS64, const ImageCheck &check = ImageCheck{},
+                         bool pipelined = false) {
   const int32_t *rows_dev = offsets + batch;
   const LnWarn lw{offsets, batch, warnings};
   int8_t *qkv = ck && ck->fused_qkv ? ck->fused_qkv : w.qkv;
@@ -234,7 +236,7 @@ static int block_forward(const hv_block_dev &p, const int8_t *x, const int32_t *
     a.qkv_shift = g.shift_a; a.qkv_acc_lim = g.acc_lim; a.bqkv_max = bias_max;
   }
   a.qkv = qkv; a.offsets = offsets; a.ctx = ctx; a.batch = batch; a.rows_cap = max_rows;
-  a.status = check.status; a.warnings = check.warnings;
+  a.status = check.status; a.warnings = check.warnings; a.pipelined = pipelined;
   a.score = ck ? ck->score : nullptr;
   a.prob = ck ? ck->prob : nullptr;
   a.score_shift = p.score_exp - 2 * p.qkv_out_exp;
@@ -731,12 +733,14 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
     // rows (or for small batches), else 64-row blocks with the launch's last
     // ones split where that evens out the CUs' work; pipelined callers,
     // whose other batches fill the CUs a launch leaves idle, keep 64.
-    const int ffn_rows = (options & HV_FWD_PIPELINED)                   ? FFN_ROWS64
+    const bool pipelined = options & HV_FWD_PIPELINED;
+    const int ffn_rows = pipelined                                      ? FFN_ROWS64
                          : few_rows(max_rows, sel > 0)                  ? FFN_ROWS16
                          : (sel > 0 || small_rows((long long)max_rows)) ? FFN_ROWS32
                                                                         : FFN_ROWS64_BALANCED;
     if ((rc = block_forward(p->blocks[blk - 1], w.xa, w.off_a, batch, max_rows, w.xb, nullptr,
-                            warnings, w.blk, s, chain, w.bias_max + 4 * (blk - 1), ffn_rows)))
+                            warnings, w.blk, s, chain, w.bias_max + 4 * (blk - 1), ffn_rows,
+                            ImageCheck{}, pipelined)))
       return rc;
     ln1_ready = next_done ? w.blk.ln : nullptr;
     if (blk == 12) final_done = next_done;

@@ -187,6 +187,7 @@ struct AttnArgs {
   const int32_t *bqkv;
   int qkv_shift, qkv_acc_lim;
   int q_split;  // workgroups per (image, head), each a range of its query tiles
+  bool pipelined;  // other batches are in flight beside this one (HV_FWD_PIPELINED)
   const unsigned *bqkv_max;  // optional: largest |bias| of bqkv (GemmArgs::bias_max)
 };
 

@@ -999,13 +999,20 @@ int launch_attention(const AttnArgs &a_in, hipStream_t s) {
   // one workgroup per CU the repeated K and V cost more than the split gives:
   // fused QKV, unpruned forward on MI355X, four waves / eight / eight split in
   // two / in four (us):
-  //    1 image 385 / 352 / 306 / 288    24 images 389 / 357 / 310 / 358
-  //   42       460 / 428 / 384 / 432    64        472 / 441 / 491 / 511
-  //   85       584 / 551 / 602 / 685   100        654 / 692 / 707 / 760
-  // Over given QKV rows K and V are only loaded, and two parts stay ahead up
-  // to 1.5 pairs per CU (96 ragged images 16.2 / 14.8 / 14.3 / 16.4, 128:
-  // 19.3 / 19.3 / 18.0 / 20.2, 256: 22.9 / 23.3 / 26.4 / 32.0).
-  const int items = a.batch * 3, cus = device_cus();
+  //    1 image 345 / 316 / 270 / 253    24 images 380 / 351 / 304 / 354 (in three 300)
+  //   42       447 / 418 / 373 / 423    64        466 / 437 / 488 / 510
+  //   85       569 / 540 / 592 / 679   100        642 / 686 / 699 / 758
+  // Over given QKV rows K and V are only loaded, and two parts stay level or
+  // ahead up to 1.5 pairs per CU (96 images of 60 to 197 tokens 13.6 / 12.6 /
+  // 11.5 / 14.4, of 197 17.6 / 19.4 / 17.5 / 17.5, 128 of 197 17.9 / 19.4 / 17.9
+  // / 20.4, 129 17.9 / 19.4 / 22.1 / 22.5).
+  // A pipelined forward's other batches fill the CUs it leaves, so there the
+  // repeated K and V cost their whole time, and it splits as if it had half the
+  // CUs.  Three unpruned batches in flight, four waves / eight / eight split in
+  // two / in four, and the split by the batch alone (us):
+  //   16 images 626 / 559 / 515 / 559, 562    24 images 651 / 592 / 598 / 654, 649
+  //   42        710 / 724 / 815 / 891, 816    85        1047 / 1159 / 1307 / 1561, 1154
+  const int items = a.batch * 3, cus = a.pipelined ? device_cus() / 2 : device_cus();
   const bool wide = a.ln1 ? items <= cus : 2 * items <= 3 * cus;
   const int nw = wide ? 8 : 4, per_cu = cus / items;
   a.q_split = !wide ? 1 : (a.ln1 ? min(max(per_cu, 1), 4) : (per_cu >= 4 ? 4 : 2));
