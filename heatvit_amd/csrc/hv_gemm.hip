@@ -777,10 +777,10 @@ static int run_lds(const GemmArgs &g, hipStream_t s) {
 template <int EPI>
 static int dispatch(const GemmArgs &g, int a_mode, hipStream_t s) {
   if constexpr (EPI == EPI_PATCH) {
-    // A from the NHWC images (gathered patches) or from patch rows [B*196][768]
-    if (g.k != 768 || (a_mode != A_PATCH && (a_mode != A_ROWS || g.lda != 768)))
+    // A from the NHWC images (gathered patches; a forward's patch rows take
+    // k_patch_init)
+    if (g.k != 768 || a_mode != A_PATCH)
       return fail(HV_EVALUE, HV_ERR_DIMENSION, "gemm: bad patch GEMM");
-    if (a_mode == A_ROWS) return run_lds<2, 1, 2, EPI_PATCH, A_ROWS, 24>(g, s);
     return run_lds<2, 1, 2, EPI_PATCH, A_PATCH, 24>(g, s);
   } else {
     if (a_mode == (A_ROWS | A_UNSIGNED)) return run<1, 1, 2, EPI, A_ROWS | A_UNSIGNED, 0>(g, s);
@@ -2068,7 +2068,8 @@ int launch_patch_embed(const hv_patch_dev &p, const int8_t *images, int batch, i
   if (init)
     return patch_rows ? launch_patch_init<A_ROWS>(g, p, *init, s)
                       : launch_patch_init<A_PATCH>(g, p, *init, s);
-  const int rc = launch_gemm(g, patch_rows ? A_ROWS : A_PATCH, EPI_PATCH, s);
+  if (patch_rows) return fail(HV_EVALUE, HV_ERR_OPCODE, "patch: rows only in a forward");
+  const int rc = launch_gemm(g, A_PATCH, EPI_PATCH, s);
   if (rc) return rc;
   hv_launch(k_cls_rows, dim3(batch), dim3(192), 0, s, p.cls, p.pos, x, p.cls_exp,
                      p.pos_exp, p.tokens_exp);

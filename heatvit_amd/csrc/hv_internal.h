@@ -116,8 +116,8 @@ int launch_gelu_post(bool table, const int64_t *in, int64_t *out, int64_t n, int
                      hipStream_t s);
 
 // Patch embedding (transformer.patch_embedding): A rows are gathered
-// patches of NHWC 224x224x3 images (or, with patch_rows, the patch matrix
-// [B*196][768] itself), epilogue adds the position rows, and the CLS rows
+// patches of NHWC 224x224x3 images (or, with patch_rows and init, the patch
+// matrix [B*196][768] itself), epilogue adds the position rows, and the CLS rows
 // are written by a second small kernel.
 // init (optional): the same launch also writes the CLS rows and a forward's
 // start: offsets [batch + 1] of HV_MAX_TOKENS rows an image, cleared package
@@ -227,7 +227,7 @@ struct SelectorArgs {
   int8_t *pkg_rows;     // workspace [B][192]: package rows (selector forward)
   int32_t *token_counts;  // optional [B][4] column `stage`
   int stage;
-  int32_t *img_warn;      // optional [B]: the state's warning bits are ORed in
+  int32_t *img_warn;      // optional [B]: the state's warning bits are ORed in (forward)
   hv_selector_ckpt ck;    // optional intermediate outputs (null pointers skip)
   const Ln32 *ln;         // optional (selector forward): also the LayerNorm of the output rows
 };
@@ -241,7 +241,6 @@ struct SelectorRows {
   int32_t *out_offsets;
   uint8_t *pkg_out;
   int32_t *token_counts;  // optional [B][4] column `stage`
-  int32_t *img_warn;      // optional [B]
   int batch, stage;
 };
 int launch_selector_rows(const SelectorRows &a, const Ln32 *ln, hipStream_t s);

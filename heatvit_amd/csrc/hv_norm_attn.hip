@@ -316,9 +316,8 @@ __global__ __launch_bounds__(256) void k_selector_rows(SelectorRows a, Ln32 ln) 
     }
     sx = group_sum<8>(sx);
     sxx = group_sum<8>(sxx);
+    // (never a negative variance: ln_rows)
     const LnRow c = ln_row_consts_e<LnEstHw>(sx, sxx, ln.s, ln.t);
-    if (live && c.neg_var && sub == 0 && a.img_warn)
-      atomicOr(&a.img_warn[b], HV_WARN_LN_NEGATIVE_VARIANCE);
     const int rnd = 1 << (ln.os - 1);
     int out[6];
     if (__any(live && c.tie)) ln32_elems24<true>(w, g, bb, c, rnd, ln.os, out);

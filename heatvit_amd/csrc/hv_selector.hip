@@ -125,10 +125,10 @@ __device__ __forceinline__ void state_invalid(int32_t *st) {
 // head statistics (3 -> 3), its PLAN layer (3 -> 3), and the weighted mean
 // of the head scores (plain mean, and the warning, when the weights sum to
 // zero).  The biases are any int32 and the reference adds them in int64
-// (gemm.py:118-119): the three products (|sum| < 2^16; weights and bias from LDS) are summed in 32
-// bits and the bias added in 64; the empty asm keeps the compiler from
-// folding bias and products into one 32-bit dot-product accumulation, which
-// wraps for biases near the int32 limits.
+// (gemm.py:118-119): the three products (|sum| < 2^16; weights and bias from
+// LDS) are summed in 32 bits and the bias added in 64; the empty asm keeps the
+// compiler from folding bias and products into one 32-bit dot-product
+// accumulation, which wraps for biases near the int32 limits.
 __device__ __forceinline__ int fuse_hidden(const hv_selector_dev &p, const int8_t *stats,
                                            const int *wt, int bias) {
   const int a_in = -16 - (p.stats_out_exp + p.hw_w1_exp), a_out = p.hw_hidden_out_exp + 16;
@@ -694,7 +694,7 @@ __global__ __launch_bounds__(kImgThreads) void k_selector_image(
 __global__ __launch_bounds__(256) void k_selector_keep(const int32_t *offsets,
                                                        const uint8_t *pkg_in, int batch,
                                                        const int32_t *fused, int32_t *kept_index,
-                                                       int32_t *state, int32_t *img_warn) {
+                                                       int32_t *state) {
   const int b = xcd_image(batch);
   if (b < 0) return;
   const int c = threadIdx.x;
@@ -708,7 +708,6 @@ __global__ __launch_bounds__(256) void k_selector_keep(const int32_t *offsets,
   const int fc = c < C ? fused[(size_t)b * kMaxCand + c] : 0;
   const bool bad = c < C && (unsigned)fc > 65536u;
   keep_list<256>(C, pkg, fc, false, bad, kept_index + (size_t)b * kMaxCand, st);
-  if (c == 0 && img_warn && st[0] > 0) img_warn[b] |= st[4];
 }
 
 // finalize_tokens' stream compaction of one image (XCD-major): the image's
@@ -718,7 +717,7 @@ __global__ __launch_bounds__(256) void k_selector_keep(const int32_t *offsets,
 __global__ __launch_bounds__(256) void k_selector_compact(
     const int8_t *tokens, const int32_t *offsets, const uint8_t *pkg_in, int batch,
     const int32_t *fused, const int32_t *kept_index, const int32_t *state,
-    int8_t *out, int32_t *out_offsets, uint8_t *pkg_out, int32_t *token_counts, int stage) {
+    int8_t *out, int32_t *out_offsets, uint8_t *pkg_out) {
   __shared__ int wgt[kMaxCand];
   __shared__ int part_sum[21 * 192];
   __shared__ int src_k[kMaxCand + 1];
@@ -739,7 +738,6 @@ __global__ __launch_bounds__(256) void k_selector_compact(
     out_offsets[b] = out0;
     if (b == batch - 1) out_offsets[batch] = out0 + max(count, 0);
     pkg_out[b] = (uint8_t)(count > 0 ? exists : 0);
-    if (token_counts) token_counts[(size_t)b * 4 + stage] = count;
   }
   if (count <= 0) return;  // uniform
   const int row0 = offsets[b], C = offsets[b + 1] - row0 - 1;
@@ -802,18 +800,17 @@ int launch_selector(const SelectorArgs &a, hipStream_t s) {
               table(p.h2_out_exp + 16), a.fused, a.kept_index, a.state, a.pkg_rows, a.img_warn);
     if ((rc = check_hip(hipGetLastError(), "k_selector_image launch"))) return rc;
     const SelectorRows rows{a.tokens, a.offsets, a.kept_index, a.state, a.pkg_rows,
-                            a.out_tokens, a.out_offsets, a.pkg_out, a.token_counts, a.img_warn,
+                            a.out_tokens, a.out_offsets, a.pkg_out, a.token_counts,
                             a.batch, a.stage};
     if (!a.ln) return launch_selector_rows(rows, nullptr, s);
     const ProfScope ps(HV_PROF_LAYERNORM, s);  // the launch it stands in for
     return launch_selector_rows(rows, a.ln, s);
   }
   hv_launch(k_selector_keep, grid, dim3(256), 0, s, a.offsets, a.pkg_in, a.batch, a.fused,
-            a.kept_index, a.state, a.img_warn);
+            a.kept_index, a.state);
   if ((rc = check_hip(hipGetLastError(), "k_selector_keep launch"))) return rc;
   hv_launch(k_selector_compact, grid, dim3(256), 0, s, a.tokens, a.offsets, a.pkg_in, a.batch,
-            a.fused, a.kept_index, a.state, a.out_tokens, a.out_offsets, a.pkg_out,
-            a.token_counts, a.stage);
+            a.fused, a.kept_index, a.state, a.out_tokens, a.out_offsets, a.pkg_out);
   return check_hip(hipGetLastError(), "k_selector_compact launch");
 }
 
