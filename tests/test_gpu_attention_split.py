@@ -33,6 +33,21 @@ def test_attention_over_given_qkv(oracle, batch):
         assert np.array_equal(got[i], want), (batch, i, len(q))
 
 
+@pytest.mark.parametrize("exponents", range(6))
+@pytest.mark.parametrize("batch", (15, 30, 129))
+def test_attention_exponents_over_given_qkv(oracle, batch, exponents):
+    """The score and context exponents of test_gpu_attention's sweep, whose
+    launches with score and prob outputs keep four wavefronts, on four parts of
+    eight, two parts, and four wavefronts without those outputs."""
+    from test_gpu_attention import EXPS, peaky_qkv
+    assert len(EXPS) == 6
+    rng = np.random.default_rng(7 * batch + exponents)
+    qkvs = [peaky_qkv(rng, n) for n in _lengths(batch)]
+    got = _context(qkvs, EXPS[exponents])
+    for i, q in enumerate(qkvs):
+        assert np.array_equal(got[i], oracle.attention(q, *EXPS[exponents])[2]), (i, len(q))
+
+
 def _context(qkvs, exps):
     """The context rows of hv_attention_i8 without score and prob outputs
     (whose launches keep four wavefronts), and its status."""

@@ -43,12 +43,13 @@ def test_block_ragged_batch_vs_oracle(oracle):
             assert np.array_equal(cks[i][k], ck[k]), (i, k)
 
 
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("wide", ["b1", "b2", "both"])
-def test_fused_ffn_wide_biases_and_ragged_rows_vs_oracle(oracle, wide):
+def test_fused_ffn_wide_biases_and_ragged_rows_vs_oracle(oracle, wide, many):
     """Without checkpoints the block's FFN runs as one fused kernel (hidden
     rows in LDS); an FFN1 or FFN2 bias beyond the int32 epilogue bound sends
     that phase to the exact 64-bit forms, and ragged images leave partial
-    64-row blocks."""
+    row blocks (of 16 rows, with many images of 32)."""
     import dataclasses
     from heatvit_amd.transformer import transformer_block_batch
     _, bp = synth.block_workload()
@@ -64,7 +65,8 @@ def test_fused_ffn_wide_biases_and_ragged_rows_vs_oracle(oracle, wide):
         b2[77] = -(1 << 30)
     bp = dataclasses.replace(bp, ffn=dataclasses.replace(bp.ffn, b1=b1, b2=b2))
     rng = np.random.default_rng(8)
-    lens = [197, 63, 1, 65, 130, 197, 7]
+    lens = RAGGED_MANY if many else [197, 63, 1, 65, 130, 197, 7]
+    _assert_dispatch(lens, many)
     xs = [rng.integers(-128, 128, (n, 192)).astype(np.int8) for n in lens]
     zs = transformer_block_batch(xs, bp)
     for i, x in enumerate(xs):
@@ -129,25 +131,47 @@ def test_fused_ffn_split_blocks_past_the_live_rows_vs_oracle(oracle):
         assert np.array_equal(zs[offsets[i]:offsets[i + 1]], want), (i, len(xi))
 
 
-# Ragged token counts of a pruned stage: partial 32-row tiles and 64-row
-# FFN blocks, images of one and two key tiles, many small images; 32 images,
-# so the attention kernel runs the QKV GEMM.
+# Ragged token counts of a pruned stage: partial row tiles and FFN blocks,
+# images of one and two key tiles, many small images; 32 images, so the
+# attention kernel runs the QKV GEMM.
 RAGGED_LENS = [1, 2, 16, 17, 31, 32, 33, 48, 63, 64, 65, 100, 128, 129, 150, 197] + [3] * 16
 
 
-def _ragged_batch(rng, lens=RAGGED_LENS):
+# The same images six times: on a 256-CU device RAGGED_LENS takes the fused
+# FFN's 16-row blocks and the attention's eight wavefronts with split queries,
+# this batch its 32-row blocks and four wavefronts.
+RAGGED_MANY = RAGGED_LENS[:16] * 6
+
+
+def _assert_dispatch(lens, many):
+    """The batch lies on its side of the dispatch's bounds: at most 16 rows and
+    one (image, head) pair per CU, or more of both and too few rows for 64-row
+    blocks."""
+    import torch
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if many:
+        assert 16 * cus < sum(lens) < 2 * 256 * 64 and 3 * len(lens) > cus
+    else:
+        assert sum(lens) <= 16 * cus and 3 * len(lens) <= cus
+
+
+def _ragged_batch(rng, lens=RAGGED_LENS, many=False):
+    if many:
+        lens = RAGGED_MANY
+    _assert_dispatch(lens, many)
     return [rng.integers(-128, 128, (n, 192)).astype(np.int8) for n in lens]
 
 
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("blk", range(12))
-def test_block_every_model_block_ragged_vs_oracle(oracle, blk):
+def test_block_every_model_block_ragged_vs_oracle(oracle, blk, many):
     """Every block of the 256-image workload's model (its requant
     directions, attention modes and GELU tables differ) over a ragged batch
-    of mostly small images, against the oracle."""
+    of mostly small images, few and many, against the oracle."""
     from heatvit_amd.transformer import transformer_block_batch
     _, params = synth.throughput_workload(1)
     bp = params.blocks[blk]
-    xs = _ragged_batch(np.random.default_rng(100 + blk))
+    xs = _ragged_batch(np.random.default_rng(100 + blk), many=many)
     zs = transformer_block_batch(xs, bp)
     for i, x in enumerate(xs):
         z, _ = oracle.transformer_block(x, bp, checkpoints=False)
@@ -178,7 +202,7 @@ def test_block_ln2_inside_fused_ffn_vs_oracle(oracle):
     keeps the QKV launch.  With checkpoints QKV, the projection and LN2 have
     launches of their own, which write the fused_qkv, y and ln2 checkpoints,
     and FFN1 / FFN2 run as two GEMMs (the hidden checkpoint).  All match the
-    oracle over ragged images (partial 32-row tiles and 64-row blocks)."""
+    oracle over ragged images (partial row tiles and blocks)."""
     _, bp = synth.block_workload()
     xs = _ragged_batch(np.random.default_rng(21))
     zs, n = _block_launches(xs, bp, False)
@@ -201,14 +225,15 @@ def test_block_ln2_inside_fused_ffn_vs_oracle(oracle):
         assert np.array_equal(cks[i]["fused_qkv"], ck["fused_qkv"]), (i, len(x))
 
 
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("msa_exp,ffn_x_exp,dirs", [(-7, -11, 0), (-13, -12, 1), (-7, -12, 2),
                                                     (-11, -12, 3)])
 def test_block_projection_requant_directions_in_ffn_kernel_vs_oracle(oracle, msa_exp,
-                                                                     ffn_x_exp, dirs):
+                                                                     ffn_x_exp, dirs, many):
     """The projection inside the fused FFN kernel with each pair of requant
     directions (bit 0: the product's requant shifts left, msa_out at or
     below context_out + wproj; bit 1: the residual align-add's output shift
-    is not positive), over 32 ragged images without checkpoints: no
+    is not positive), over 32 and 96 ragged images without checkpoints: no
     projection launch, and z equal to the oracle's."""
     import dataclasses
     _, bp = synth.block_workload()
@@ -218,7 +243,7 @@ def test_block_projection_requant_directions_in_ffn_kernel_vs_oracle(oracle, msa
     assert (shift_a <= 0) + 2 * (os_ <= 0) == dirs
     bp = dataclasses.replace(bp, mhsa=dataclasses.replace(m, msa_out_scale_exp=msa_exp),
                              ffn=dataclasses.replace(f, x_scale_exp=ffn_x_exp))
-    xs = _ragged_batch(np.random.default_rng(40 + dirs))
+    xs = _ragged_batch(np.random.default_rng(40 + dirs), many=many)
     zs, n = _block_launches(xs, bp, False)
     assert n["gemm_proj"] == 0 and n["ffn"] == 1 and n["layernorm"] == 1, n
     for i, x in enumerate(xs):
@@ -226,10 +251,11 @@ def test_block_projection_requant_directions_in_ffn_kernel_vs_oracle(oracle, msa
         assert np.array_equal(zs[i], z), (i, len(x))
 
 
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("qkv_exp,score_exp", [(-9, -21), (-4, -11), (-9, -7), (-19, -30)])
-def test_block_attention_with_qkv_in_kernel_exponents_vs_oracle(oracle, qkv_exp, score_exp):
-    """The QKV GEMM inside the attention kernel over 32 ragged images without
-    checkpoints, under the score paths of the int32 Q8.16 conversion (a
+def test_block_attention_with_qkv_in_kernel_exponents_vs_oracle(oracle, qkv_exp, score_exp, many):
+    """The QKV GEMM inside the attention kernel over 32 and 96 ragged images
+    (eight wavefronts and four) without checkpoints, under the score paths of the int32 Q8.16 conversion (a
     right shift, a plain saturation, the general two-step form) and a QKV
     requant that shifts left (the last case): no QKV launch, z equal to the
     oracle's."""
@@ -237,7 +263,7 @@ def test_block_attention_with_qkv_in_kernel_exponents_vs_oracle(oracle, qkv_exp,
     _, bp = synth.block_workload()
     bp = dataclasses.replace(bp, mhsa=dataclasses.replace(
         bp.mhsa, qkv_out_scale_exp=qkv_exp, score_scale_exp=score_exp))
-    xs = _ragged_batch(np.random.default_rng(60 - qkv_exp))
+    xs = _ragged_batch(np.random.default_rng(60 - qkv_exp), many=many)
     zs, n = _block_launches(xs, bp, False)
     assert n["gemm_qkv"] == 0 and n["attention"] == 1, n
     for i, x in enumerate(xs):
@@ -245,7 +271,8 @@ def test_block_attention_with_qkv_in_kernel_exponents_vs_oracle(oracle, qkv_exp,
         assert np.array_equal(zs[i], z), (i, len(x))
 
 
-def test_block_wide_biases_all_gemms_vs_oracle(oracle):
+@pytest.mark.parametrize("many", [False, True])
+def test_block_wide_biases_all_gemms_vs_oracle(oracle, many):
     """Biases beyond the int32 epilogue bounds in all four GEMMs send their
     tiles to the exact 64-bit forms (the projection's inside the fused FFN
     kernel, as the block runs without checkpoints)."""
@@ -260,7 +287,7 @@ def test_block_wide_biases_all_gemms_vs_oracle(oracle):
     b2[[0, 100]] = [-(1 << 31), (1 << 31) - 1]
     bp = dataclasses.replace(bp, mhsa=dataclasses.replace(bp.mhsa, bqkv=bqkv, bproj=bproj),
                              ffn=dataclasses.replace(bp.ffn, b1=b1, b2=b2))
-    xs = _ragged_batch(np.random.default_rng(9))
+    xs = _ragged_batch(np.random.default_rng(9), many=many)
     zs = transformer_block_batch(xs, bp)
     for i, x in enumerate(xs):
         z, _ = oracle.transformer_block(x, bp, checkpoints=False)
@@ -497,6 +524,84 @@ def test_model_layernorm_fallbacks_vs_oracle(oracle):
     assert not status.any()
     assert np.array_equal(r.logits, logits)
     assert np.array_equal(r.token_counts, counts)
+    assert np.array_equal(r.warnings, warnings)
+
+
+def test_model_layernorm_after_selector_falls_back_vs_oracle(oracle):
+    """Blocks 4 and 10, the first behind a selector, with LayerNorm 1 outside
+    the int32 form: those selectors' compactions then write no LayerNorm (the
+    profiler counts them as selector launches) and the general kernel runs;
+    block 7's stays in its compaction."""
+    import dataclasses
+    from heatvit_amd import _lib
+    from heatvit_amd.model import HeatViTModel
+    imgs, params = synth.pruned_workload(6)
+    blocks = list(params.blocks)
+    for i in (3, 9):
+        m = blocks[i].mhsa
+        blocks[i] = dataclasses.replace(
+            blocks[i], mhsa=dataclasses.replace(m, beta1_scale_exp=m.gamma1_scale_exp - 17))
+    p = dataclasses.replace(params, blocks=tuple(blocks))
+    L = _lib.lib()
+    L.hv_profile_enable(1)
+    try:
+        r = HeatViTModel().infer_batch(imgs, p)
+        ms = np.zeros(len(_lib.PROF_CLASSES), np.float32)
+        n = np.zeros(len(_lib.PROF_CLASSES), np.int32)
+        _lib.check(L.hv_profile_read(ms.ctypes.data, n.ctypes.data, len(ms)), "profile")
+    finally:
+        L.hv_profile_enable(0)
+    n = dict(zip(_lib.PROF_CLASSES, n.tolist()))
+    assert n["selector"] == 3 + 2 and n["layernorm"] == 2 + 2, n
+    logits, counts, status, warnings = oracle.model_infer_batch(imgs, p)
+    assert not status.any()
+    assert np.array_equal(r.logits, logits)
+    assert np.array_equal(r.token_counts, counts)
+    assert np.array_equal(r.warnings, warnings)
+
+
+# (activation, tokens, pos) exponents, the pair of requant directions (bit 0:
+# the product's shifts left, bit 1: the align-add's) or None: 24 binary places
+# between activation and pos leave the int32 epilogue
+PATCH_EXPS = [(-7, -5, -4, 0), (-18, -5, -4, 1), (-7, -9, -4, 2), (-15, -16, -4, 3),
+              (-7, -5, -31, None)]
+
+
+@pytest.mark.parametrize("floats", [False, True])
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("act,tok,pos,dirs", PATCH_EXPS)
+def test_model_patch_epilogues_vs_oracle(oracle, act, tok, pos, dirs, wide, floats):
+    """The forward's own patch launch (patch GEMM, CLS rows and the forward's
+    start) with each pair of requant directions and the exact epilogue, wide:
+    biases at the ends of int32, from int8 images (gathered) and float ones
+    (patch rows); one tile of 128 rows and a partial one per image."""
+    import dataclasses
+    from heatvit_amd.model import HeatViTModel
+    imgs, params = synth.pruned_workload(3)
+    pp = params.patch
+    if dirs is None:
+        assert abs(act - pos) > 21
+    else:
+        assert (act <= pp.image_scale_exp + pp.weight_scale_exp) + 2 * (tok <= min(act, pos)) \
+            == dirs
+    bias = np.asarray(pp.patch_bias).astype(np.int64).copy()
+    if wide:
+        bias[[0, 77, 191]] = [(1 << 31) - 1, -(1 << 31), 1 << 30]
+    pp = dataclasses.replace(pp, activation_scale_exp=act, tokens_scale_exp=tok,
+                             pos_scale_exp=pos, patch_bias=bias)
+    p = dataclasses.replace(synth.unpruned_control(params), patch=pp)
+    m = HeatViTModel()
+    if floats:
+        x = imgs.reshape(-1, 224, 224, 3).transpose(0, 3, 1, 2).astype(np.float32)
+        r = m.infer_float_batch(np.ascontiguousarray(x * 2.0 ** pp.image_scale_exp), p,
+                                checkpoints=True)
+    else:
+        r = m.infer_batch(imgs, p, checkpoints=True)
+    for i in range(3):
+        assert np.array_equal(r.checkpoints[i]["patch"], oracle.patch_embedding(imgs[i], pp)), i
+    logits, _, status, warnings = oracle.model_infer_batch(imgs, p)
+    assert not status.any()
+    assert np.array_equal(r.logits, logits)
     assert np.array_equal(r.warnings, warnings)
 
 
