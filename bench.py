@@ -62,15 +62,17 @@ def class_work(counts, params, batch):
     patch; head 2*192*1000 per image; selector 2*13938 per candidate.  The
     attention kernel computes its head's Q, K and V itself (the LayerNorm 1
     rows in, the context rows out: 384 B per token, with the QKV ops); where
-    the QKV GEMM runs as its own launch instead (fewer than 32 images),
-    `launched_work` moves those ops back to it.  The fused FFN kernel runs
+    the QKV GEMM runs as its own launch instead (a block call of fewer than 32
+    images), `launched_work` moves those ops back to it.  The fused FFN kernel runs
     the attention projection and its residual (the context rows and x in
     once; y stays on the CU), LayerNorm 2, FFN1,
     FFN2 and writes the block output and, when the next block follows
     without a selector in between, that block's LayerNorm 1 (block 12: the
-    final LayerNorm): 576 B per token plus 192 B for those blocks; the
-    LayerNorm class is then each stage's first LayerNorm 1.  Only the
-    classes a run launches are reported."""
+    final LayerNorm): 576 B per token plus 192 B for those blocks.  The
+    LayerNorm class is then block 1's LayerNorm 1 and, behind each selector,
+    the compaction that also writes one (the kept rows in, rows and LayerNorm
+    out); the selector class is the selector kernel alone (its token rows in).
+    Only the classes a run launches are reported."""
     counts = np.asarray(counts, np.int64)
     stage_of_block = []
     s = 0

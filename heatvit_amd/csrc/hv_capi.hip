@@ -167,7 +167,8 @@ static bool few_rows(long long rows, bool pruned) {
 }
 
 // Images per batch from which hv_block_forward's attention kernel runs the
-// QKV GEMM (the model's does at every batch size).
+// QKV GEMM (the model's does at every batch size); block_forward has both sides
+// measured.
 static constexpr int kFusedQkvMinBatch = 32;
 
 // transformer_block (transformer.py:401-431) on rows [0, offsets[batch]):
@@ -216,10 +217,11 @@ static int block_forward(const hv_block_dev &p, const int8_t *x, const int32_t *
   // Without checkpoints the attention kernel computes each head's Q, K and
   // V itself when their requant takes the int32 form: qkv never reaches
   // memory, and a launch is saved (one image, unpruned forward: 288 us with
-  // it in the kernel, 309 us with the separate GEMM).  A block call of few
-  // images has no tensor-wide bias bound, so its in-kernel requant would vote
-  // tile by tile, and keeps the separate GEMM (one image: 27.0 us, 25.7 us
-  // in the kernel).
+  // it in the kernel, 309 us with the separate GEMM).  Block calls of fewer
+  // than kFusedQkvMinBatch images keep the launch that their profiles show as
+  // gemm_qkv, although it costs them (us with it, and in the kernel): 1 image
+  // of 197 tokens 23.9, 21.6, 16 images 24.8, 22.7, 31 images 28.1, 25.5, of 60
+  // tokens 23.0, 20.0.
   epilogue_limits_pub(g, HV_EPI_I8);
   const bool fuse_qkv = !ck && (bias_max || batch >= kFusedQkvMinBatch) && g.narrow_ok && g.shift_a >= -30 &&
                         g.shift_a <= 30 &&
@@ -729,10 +731,11 @@ static int model_forward(const hv_model_dev *p, const void *images, bool float_i
     bool next_done = false;
     const LnChain chain{ln1_ready, chain_next ? (blk < 12 ? &p->blocks[blk] : &fin) : nullptr,
                         w.blk.ln, &next_done};
-    // One forward at a time, 32-row FFN blocks once a selector has cut the
-    // rows (or for small batches), else 64-row blocks with the launch's last
-    // ones split where that evens out the CUs' work; pipelined callers,
-    // whose other batches fill the CUs a launch leaves idle, keep 64.
+    // One forward at a time, 16-row FFN blocks for few rows, 32-row ones once
+    // a selector has cut the rows (or for small batches), else 64-row blocks
+    // with the launch's last ones split where that evens out the CUs' work;
+    // pipelined callers, whose other batches fill the CUs a launch leaves
+    // idle, keep 64.
     const bool pipelined = options & HV_FWD_PIPELINED;
     const int ffn_rows = pipelined                                      ? FFN_ROWS64
                          : few_rows(max_rows, sel > 0)                  ? FFN_ROWS16

@@ -819,9 +819,10 @@ __device__ __forceinline__ void attn_tiles(const AttnArgs &g, const int8_t *Ks, 
   }
 }
 
-// At most 168 VGPRs (three workgroups per CU): the 768 items of a 256-image
-// batch then run in one round.  FQ: fused QKV (qkv_head), FQL its requant
-// shifting left.
+// FQ: fused QKV, FQL its requant shifting left.  NW = 4: at most 168 VGPRs, so
+// three workgroups fit a CU and the 768 items of a 256-image batch run in one
+// round.  NW = 8: 160 VGPRs are three wavefronts per SIMD, one workgroup per
+// CU, so launch_attention's split stays within one per CU.
 template <int MODE, bool CKPT, bool FQ, bool FQL, int NW>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 3 : 2) void k_attention(AttnArgs g) {
   constexpr int NTH = 64 * NW;
@@ -1049,7 +1050,7 @@ int launch_attention(const AttnArgs &a_in, hipStream_t s) {
 // 65554), so their reciprocal takes the 32-bit form; longer rows the 64-bit
 // one.  att / sel may be NULL.
 // The path is bound by memory: 151,296 rows of 197 (119 MB in, 30 MB out)
-// take 29.0 us, 5.1 TB/s, where a large copy reaches 4.9.  One wavefront per
+// take 29.0 us, 5.1 TB/s, the rate of a 1 GiB copy (256 MiB: 5.4).  One wavefront per
 // row with 4-byte loads and byte stores took 62.6 us (a division by a
 // constant per entry, 24 shuffles per row).
 // ---------------------------------------------------------------------------

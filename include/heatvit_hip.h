@@ -400,6 +400,17 @@ int hv_model_forward_f32_ex(const hv_model_dev *p, const float *images, int batc
 /* returns the summed milliseconds and launch counts per class (arrays   */
 /* of n entries), then clears the record.  Not thread-safe: one          */
 /* profiling client at a time.                                           */
+/*                                                                       */
+/* A launch counts in one class, whatever other work it carries:         */
+/* PATCH: the patch GEMM with the forward's start (offsets, CLS rows,    */
+/* flags, bias bounds) and, for float images, the quantiser.             */
+/* LAYERNORM: LayerNorm launches, and the compaction behind a selector   */
+/* where it also writes the next block's LayerNorm 1 (its row copies     */
+/* included).  SELECTOR: the selector proper, and its compaction where   */
+/* that writes no LayerNorm.  ATTENTION: with the QKV GEMM when no       */
+/* GEMM_QKV launch ran.  FFN: with the projection, the LayerNorm in      */
+/* front of it and the next one where those have no launches.  OTHER:    */
+/* no launch of a forward.                                               */
 /* ------------------------------------------------------------------ */
 
 #define HV_PROF_PATCH 0
@@ -412,7 +423,7 @@ int hv_model_forward_f32_ex(const hv_model_dev *p, const float *images, int batc
 #define HV_PROF_SELECTOR 7
 #define HV_PROF_HEAD 8
 #define HV_PROF_OTHER 9
-#define HV_PROF_FFN 10 /* FFN1 + GELU + FFN2 + residual in one kernel */
+#define HV_PROF_FFN 10
 #define HV_PROF_CLASSES 11
 
 int hv_profile_enable(int on);
